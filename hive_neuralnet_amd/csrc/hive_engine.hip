@@ -11,6 +11,7 @@
 #include "../../include/hive_gpu.h"
 #include "hive_leaf.hpp"
 #include "hive_phases.hpp"
+#include "hive_succ.hpp"
 
 using namespace hw;
 
@@ -192,43 +193,33 @@ __global__ __launch_bounds__(64) void k_actions(const uint8_t* __restrict__ stat
 // a zero state and move for rows that reference no valid (root, move)
 __device__ __attribute__((aligned(16))) const uint8_t kZeroRow[kStateBytes] = {};
 
-// rows of successor features per lane group: consecutive rows of one root
-// share the root's load
-constexpr int kSuccRows = 8;
-constexpr int64_t kSuccGrid = 16384;  // workgroups of the successor kernels (they stride beyond)
-// register budget of the successor kernels, by index type: the 32-bit row
-// arithmetic fits 6 waves per SIMD (80 VGPRs, no spills; the LDS boards of
-// 24 workgroups fill a CU's 160 KB), the 64-bit one 5 (96 VGPRs; at 80 it
-// spills); left alone the row loop takes ~109
-template <typename Ix>
-constexpr int kSuccWaves = sizeof(Ix) == 4 ? 6 : 5;
+// Successor kernels: how many workgroups they launch (a multiple of the 256
+// CUs; 18 workgroups' LDS boards fill a CU's 160 KB) and the register budget
+// that lets that many run (4 waves per SIMD).
+constexpr int64_t kSuccGrid = 256 * 16;
+constexpr int kSuccWaves = 4;
+// rows per block: a kSuccSpread-th of the batch, from kSuccShort to kSuccBlock
+constexpr int kSuccShort = 8, kSuccBlock = 32, kSuccSpread = 2048;
+// Batches of at most kSuccStream rows go row by row, a lane group each
+// (successor_row): one row takes about a third of a pass's time.  Leaf
+// evaluation by rows / by passes, us: mid-game base game 14 K rows 65 / 73,
+// 27 K 88 / 76, 53 K 133 / 94; every piece 9 K rows 77 / 96, 19 K 104 / 102,
+// 38 K 155 / 110; after two plies 15 K 61 / 60, 31 K 73 / 61
+constexpr int kSuccStream = 18432;
+// lane groups a batch of leaves is spread over by cutting its lists into parts
+constexpr int kSuccParts = 8, kSuccTarget = 8192;
 
-// Row blocks of R rows: lane group q of the grid takes blocks q,
-// q + 2 * gridDim.x, ... one row after another, as one stream (a root's
-// board carries over a block boundary).  R = kSuccRows when every lane group
-// of the grid has that many rows to do, fewer when the rows are few (down to
-// one row per group: the count is known only on the device, and a short
-// batch is bound by the latency of each group's rows in series, not by the
-// board loads that longer runs share).  The loop count is uniform over the
-// workgroup: both groups run while the first group's block is in range.
-template <typename Ix>
-HW_INL void successor_stream(const uint8_t* __restrict__ states, const uint8_t* __restrict__ legal,
-                             const int64_t* __restrict__ a2r, const int64_t* __restrict__ midx, Ix N,
-                             int64_t num_roots, float* __restrict__ feat_out) {
-    __shared__ Pos PS[kPosPerWave];
-    const int grp = threadIdx.x >> 5;
-    const Ix groups = (Ix)kPosPerWave * (Ix)gridDim.x;
-    const Ix per = (N + groups - 1) / groups;
-    const int R = per < 1 ? 1 : (per > kSuccRows ? kSuccRows : (int)per);
-    const Ix blocks = (N + R - 1) / R;
-    SuccessorStream st;
-    for (Ix p = blockIdx.x; kPosPerWave * p < blocks; p += gridDim.x) {
-        for (int k = 0; k < R; k++) {
-            const int lane = hw_opaque(threadIdx.x);
-            const Ix i = (kPosPerWave * p + grp) * R + k;
-            successor_row<Ix>(PS[grp], st, states, legal, a2r, midx, i, N, num_roots, kZeroRow, lane, feat_out);
-        }
-    }
+// Parts that the list of each of T leaves is cut into.
+__host__ __device__ inline int successor_parts(int64_t T) {
+    const int64_t p = T > 0 ? kSuccTarget / T : 1;
+    return p < 2 ? 2 : (p > kSuccParts ? kSuccParts : (int)p);
+}
+
+// The direction and exit tables into LDS, once per workgroup (read after the first board's barriers).
+HW_INL void load_succ_tables(SuccTables& K) {
+    static_assert(sizeof(SuccTables) <= 2 * 64, "two bytes per lane");
+    for (int i = threadIdx.x; i < (int)sizeof(SuccTables); i += 64)
+        reinterpret_cast<uint8_t*>(&K)[i] = reinterpret_cast<const uint8_t*>(&kSuccTables)[i];
 }
 
 // 32-bit row arithmetic is exact when every state, move and feature offset of
@@ -238,15 +229,54 @@ inline bool successor_narrow(int64_t rows_cap, int64_t num_roots) {
            num_roots <= ((int64_t)1 << 32) / kStateBytes && num_roots <= ((int64_t)1 << 32) / (kMaxLegal * 6);
 }
 
-// fnn_successor_features_kernel (game_logic.cu:182-229): kSuccRows (root, move)
-// rows per lane group, two groups per wave, the grid striding over the rows.
+// fnn_successor_features_kernel (game_logic.cu:182-229) over rows in any
+// order: the batch in blocks of rows, one per lane group in turn.  A block
+// works out the children of each root it meets together, so longer blocks
+// meet fewer roots twice; shorter ones spread a small batch over the chip.
+// 107 K mid-game rows: blocks of 24 rows 97 us, 32 rows 96 us, blocks of 48
+// moved to the roots' first rows 135 us (their longest waves take two whole
+// roots).
 template <typename Ix>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves<Ix>))) void k_successor_features(const uint8_t* __restrict__ states,
-                                                           const uint8_t* __restrict__ legal,
-                                                           const int64_t* __restrict__ a2r,
-                                                           const int64_t* __restrict__ midx, int64_t N,
-                                                           int64_t num_roots, float* __restrict__ feat_out) {
-    successor_stream<Ix>(states, legal, a2r, midx, (Ix)N, num_roots, feat_out);
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))) void k_successor_features(
+    const uint8_t* __restrict__ states, const uint8_t* __restrict__ legal, const int64_t* __restrict__ a2r,
+    const int64_t* __restrict__ midx, int64_t n_rows, int64_t num_roots, float* feat_out) {
+    __shared__ SuccBoard GS[kPosPerWave];
+    __shared__ SuccTables K;
+    load_succ_tables(K);
+    const int lane = threadIdx.x, grp = lane >> 5;
+    const Ix N = (Ix)n_rows, groups = (Ix)kPosPerWave * (Ix)gridDim.x;
+    Ix R = N / (Ix)kSuccSpread;
+    R = R < (Ix)kSuccShort ? (Ix)kSuccShort : (R > (Ix)kSuccBlock ? (Ix)kSuccBlock : R);
+    const Ix blocks = (N + R - 1) / R;
+    auto range = [&](Ix p, Ix& lo, Ix& hi) {
+        const Ix q = p + (Ix)grp;
+        lo = q * R < N ? q * R : N;
+        hi = lo + R < N ? lo + R : N;
+    };
+    bool marks = true;
+    const bool every = N <= (Ix)kSuccStream;
+    Ix lo = 0, hi = 0;
+    if (every) {
+        const Ix per = (N + groups - 1) / groups;
+        lo = ((Ix)kPosPerWave * (Ix)blockIdx.x + (Ix)grp) * per;
+        lo = lo < N ? lo : N;
+        hi = lo + per < N ? lo + per : N;
+    } else {
+        bool general = false;
+        for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < blocks; p += groups) {
+            range(p, lo, hi);
+            general |= successor_range<Ix>(GS[grp], K, states, legal, MapRows{a2r, midx}, lo, hi, num_roots, kZeroRow,
+                                           lane, feat_out);
+        }
+        __syncthreads();  // the marks, read by other lanes
+        marks = hw_wave_any(general);
+    }
+    if (!marks) return;
+    for (Ix p = (Ix)kPosPerWave * blockIdx.x; every || p < blocks; p += groups) {
+        if (!every) range(p, lo, hi);
+        general_range<Ix>(GS[grp], states, legal, a2r, midx, lo, hi, num_roots, kZeroRow, lane, feat_out, every);
+        if (every) break;
+    }
 }
 
 __global__ __launch_bounds__(64) void k_queen_escape(const uint8_t* __restrict__ states, int64_t B,
@@ -599,9 +629,7 @@ __global__ void k_mask_scatter(const int32_t* __restrict__ actions, const int32_
 // count stays on the device.  k_rows_offsets: exclusive prefix of the
 // clamped legal counts (one workgroup, chunks of 4,096 with a running carry)
 // and the total; k_rows_map: row -> (leaf, slot); k_successor_rows: the
-// successor features of rows < total, kSuccRows per lane group, the grid
-// striding over the rows (sized from the capacity, the count read on the
-// device).
+// successor features of each leaf's rows.
 __global__ __launch_bounds__(1024) void k_rows_offsets(const int32_t* __restrict__ nlegal, int64_t T,
                                                         int64_t* __restrict__ offsets, int64_t* __restrict__ total) {
     // chunks of 4,096 counts, four consecutive counts per thread, with a
@@ -662,14 +690,64 @@ __global__ __launch_bounds__(256) void k_rows_plan(const int32_t* __restrict__ n
     rows_plan_block(nlegal, T, offsets, total, a2r, mi, (int)blockIdx.x);
 }
 
+// The rows of each leaf by one lane group, cut where that balances: with few
+// leaves into equal parts of at least kSuccShort rows, so that the chip has
+// work enough to hide a pass's latency; with many after one window's rows --
+// the launch ends with its longest waves, and the lists that need a second
+// window (a fifth of the mid-game ones) are other lane groups' work.
 template <typename Ix>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves<Ix>))) void k_successor_rows(const uint8_t* __restrict__ states,
-                                                       const uint8_t* __restrict__ legal,
-                                                       const int64_t* __restrict__ a2r,
-                                                       const int64_t* __restrict__ midx,
-                                                       const int64_t* __restrict__ total, int64_t num_roots,
-                                                       float* __restrict__ feat_out) {
-    successor_stream<Ix>(states, legal, a2r, midx, (Ix)*total, num_roots, feat_out);
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))) void k_successor_rows(
+    const uint8_t* __restrict__ states, const uint8_t* __restrict__ legal, const int64_t* __restrict__ a2r,
+    const int64_t* __restrict__ midx, const int64_t* __restrict__ offsets, int64_t T, float* feat_out) {
+    __shared__ SuccBoard GS[kPosPerWave];
+    __shared__ SuccTables K;
+    const int lane = threadIdx.x, grp = lane >> 5;
+    const int parts = successor_parts(T);
+    const int64_t items = T * parts, stride = (int64_t)kPosPerWave * gridDim.x;
+    ListRows src{0, 0};
+    auto range = [&](int64_t p, Ix& lo, Ix& hi) {
+        const int64_t q = p + grp;
+        lo = hi = 0;
+        if (q < items) {  // offsets[T] is the batch's row count
+            const int part = (int)(q / T);
+            const int64_t t = q - (int64_t)part * T;
+            const Ix o = (Ix)offsets[t], n = (Ix)offsets[t + 1] - o;
+            Ix per = (n + (Ix)parts - 1) / (Ix)parts;
+            const Ix least = parts == 2 ? (Ix)kWinRows : (Ix)kSuccShort;
+            per = per < least ? least : per;
+            const Ix a = (Ix)part * per, b = a + per;
+            lo = o + (a < n ? a : n);
+            hi = o + (b < n ? b : n);
+            src = ListRows{t, (int64_t)o};
+        }
+    };
+    bool marks = true, every = false, ready = false;
+    Ix lo = 0, hi = 0;
+    const Ix N = (Ix)offsets[T];
+    if (N <= (Ix)kSuccStream) {  // rows dealt to the lane groups, one or two each
+        const Ix groups = (Ix)kPosPerWave * (Ix)gridDim.x, per = (N + groups - 1) / groups;
+        lo = ((Ix)kPosPerWave * (Ix)blockIdx.x + (Ix)grp) * per;
+        lo = lo < N ? lo : N;
+        hi = lo + per < N ? lo + per : N;
+        every = true;
+    } else {
+        bool general = false;
+        for (int64_t p = (int64_t)kPosPerWave * blockIdx.x; p < items; p += stride) {
+            range(p, lo, hi);
+            if (!hw_wave_any(lo < hi)) continue;
+            if (!ready) load_succ_tables(K);
+            ready = true;
+            general |= successor_range<Ix>(GS[grp], K, states, legal, src, lo, hi, T, kZeroRow, lane, feat_out);
+        }
+        __syncthreads();  // the marks, read by other lanes
+        marks = hw_wave_any(general);
+    }
+    if (!marks) return;
+    for (int64_t p = (int64_t)kPosPerWave * blockIdx.x; every || p < items; p += stride) {
+        if (!every) range(p, lo, hi);
+        general_range<Ix>(GS[grp], states, legal, a2r, midx, lo, hi, T, kZeroRow, lane, feat_out, every);
+        if (every) break;
+    }
 }
 
 inline int grid_for(int64_t n, int block) { return (int)((n + block - 1) / block); }
@@ -809,7 +887,8 @@ int hg_fnn_successor_features(const uint8_t* states, const uint8_t* legal_moves,
                               const int64_t* action_to_root, const int64_t* move_indices, int64_t N, float* features,
                               void* stream) {
     if (N <= 0) return 0;
-    const int64_t pairs = (N + kSuccRows * kPosPerWave - 1) / (kSuccRows * kPosPerWave);
+    const int64_t each = N <= kSuccStream ? kPosPerWave : kSuccShort * kPosPerWave;
+    const int64_t pairs = (N + each - 1) / each;
     const dim3 grid((unsigned)(pairs < kSuccGrid ? pairs : kSuccGrid));
     if (successor_narrow(N, num_roots))
         hipLaunchKernelGGL(k_successor_features<uint32_t>, grid, dim3(64), 0, (hipStream_t)stream, states, legal_moves,
@@ -890,14 +969,18 @@ int successor_rows_plan_large(const int32_t* num_legal, int64_t T, void* workspa
 int successor_rows_after_plan(const uint8_t* states, const uint8_t* legal_moves, int64_t T, void* workspace,
                               float* features, hipStream_t s) {
     const RowsPlan R = rows_plan_of(workspace, T);
-    const int64_t pairs = (T * kMaxLegal + kSuccRows * kPosPerWave - 1) / (kSuccRows * kPosPerWave);
-    const unsigned grid = (unsigned)(pairs < kSuccGrid ? pairs : kSuccGrid);
+    // every part of every leaf, and for a small batch a lane group per row (at
+    // most 256 a leaf); workgroups with nothing to do end at once
+    int64_t pairs = (T * successor_parts(T) + kPosPerWave - 1) / kPosPerWave;
+    const int64_t streams = T * kMaxLegal / kPosPerWave < kSuccGrid ? T * kMaxLegal / kPosPerWave : kSuccGrid;
+    pairs = pairs < streams ? streams : pairs;
+    const unsigned grid = (unsigned)(pairs < 16 * kSuccGrid ? pairs : 16 * kSuccGrid);
     if (successor_narrow(T * kMaxLegal, T))  // at most 256 rows per leaf
         hipLaunchKernelGGL(k_successor_rows<uint32_t>, dim3(grid), dim3(64), 0, s, states, legal_moves, R.a2r, R.mi,
-                           R.total, T, features);
+                           R.offsets, T, features);
     else
         hipLaunchKernelGGL(k_successor_rows<int64_t>, dim3(grid), dim3(64), 0, s, states, legal_moves, R.a2r, R.mi,
-                           R.total, T, features);
+                           R.offsets, T, features);
     return finish();
 }
 

@@ -107,13 +107,6 @@ HW_INL int lone_empty_cell(const Pos& P, int target) {
     return step(q, __ffs(e) - 1);
 }
 
-// hex distance between two cells of the 23x23 grid
-__device__ __forceinline__ int hex_distance(int a, int b) {
-    const int ra = row_of(a), rb = row_of(b);
-    const int dq = (b - rb * kGrid) - (a - ra * kGrid), dr = rb - ra, ds = -(dq + dr);
-    return max(max(abs(dq), abs(dr)), abs(ds));
-}
-
 // The pieces whose move to cell `stop` could win for the mover: the move's
 // result (the opponent queen's sixth neighbour filled, the mover's own queen
 // not surrounded with it) decides before any search, and the pieces that

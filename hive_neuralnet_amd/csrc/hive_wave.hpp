@@ -87,6 +87,13 @@ __device__ __forceinline__ int step(int c, int d) { return c + win_ofs(d) - 23; 
 // (c * 2850) >> 16 equals c / 23 over that whole range)
 __device__ __forceinline__ int row_of(int c) { return (int)(((uint32_t)c * 2850u) >> 16); }
 
+// hex distance between two cells of the 23x23 grid
+__device__ __forceinline__ int hex_distance(int a, int b) {
+    const int ra = row_of(a), rb = row_of(b);
+    const int dq = (b - rb * kGrid) - (a - ra * kGrid), dr = rb - ra, ds = -(dq + dr);
+    return max(max(abs(dq), abs(dr)), abs(ds));
+}
+
 // directions whose neighbour is on the 23x23 grid
 __device__ __forceinline__ uint32_t grid6(int c) {
     int r = row_of(c), col = c - r * kGrid;

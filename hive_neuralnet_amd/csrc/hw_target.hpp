@@ -47,3 +47,10 @@ typedef uint32_t u32x4 __attribute__((vector_size(16), aligned(4)));
 #else
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
 #endif
+
+// two floats stored together (8-byte access, 4-byte alignment)
+#ifdef HW_HOST_EMU
+typedef float f32x2 __attribute__((vector_size(8), aligned(4)));
+#else
+typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+#endif

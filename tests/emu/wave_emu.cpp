@@ -5,11 +5,13 @@
 // used by tests/test_emu_engine.py to check the device logic on the CPU and
 // to debug it there.
 #define HW_HOST_EMU 1
+#include <algorithm>
 #include <memory>
 #include <thread>
 #include <vector>
 
 #include "../../hive_neuralnet_amd/csrc/hive_probe.hpp"
+#include "../../hive_neuralnet_amd/csrc/hive_succ.hpp"
 
 using namespace hw;
 
@@ -42,6 +44,7 @@ void run_group(int threads, int64_t count, F&& body) {
 }
 static Pos g_pos[kPosPerWave];
 static Replies g_rep[kPosPerWave];
+static SuccBoard g_succ[kPosPerWave];
 }  // namespace
 
 extern "C" {
@@ -78,6 +81,23 @@ void emu_successor_rows(const uint8_t* states, const uint8_t* legal, const int64
     run_group(64, (blocks + kPosPerWave - 1) / kPosPerWave * 4, [&](int64_t r, int t) {
         int64_t q = (r / 4) * kPosPerWave + t / kW;
         successor_row(g_pos[t / kW], st[t], states, legal, a2r, midx, q * 4 + r % 4, N, num_roots, zero_row, t, feat);
+    });
+}
+// The unit program (hive_succ.hpp) over rows cut into ranges of `per` rows,
+// two ranges side by side as the kernels' two lane groups take them.
+void emu_successor_units(const uint8_t* states, const uint8_t* legal, const int64_t* a2r, const int64_t* midx,
+                         int64_t N, int64_t num_roots, int64_t per, float* feat) {
+    static const uint8_t zero_row[kStateBytes] = {};
+    memset(g_succ, 0xA5, sizeof g_succ);  // LDS starts with arbitrary contents
+    const int64_t ranges = (N + per - 1) / per;
+    run_group(64, (ranges + kPosPerWave - 1) / kPosPerWave, [&](int64_t r, int t) {
+        const int64_t q = r * kPosPerWave + t / kW;
+        const int64_t lo = std::min(N, q * per), hi = std::min(N, lo + per);
+        const bool general = successor_range<int64_t>(g_succ[t / kW], kSuccTables, states, legal,
+                                                      MapRows{a2r, midx}, lo, hi, num_roots, zero_row, t, feat);
+        __syncthreads();
+        if (hw_wave_any(general))
+            general_range<int64_t>(g_succ[t / kW], states, legal, a2r, midx, lo, hi, num_roots, zero_row, t, feat);
     });
 }
 // k_random_play's ply loop with given choices: game i's board is loaded

@@ -229,6 +229,67 @@ def test_emulated_successor_rows_whole_lists(emu, oracle):
     assert np.array_equal(f.view(np.uint32), want.view(np.uint32))
 
 
+def _all_rows(n):
+    roots = np.concatenate([np.full(int(k), i, np.int64) for i, k in enumerate(n)])
+    return roots, np.concatenate([np.arange(int(k), dtype=np.int64) for k in n])
+
+
+def _units(emu, st, mv, roots, idx, per):
+    f = np.full((len(roots), 122), np.nan, np.float32)
+    emu.emu_successor_units(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
+                            ctypes.c_int64(st.shape[0]), ctypes.c_int64(per), _p(f))
+    return f
+
+
+@pytest.mark.parametrize("mask,max_ply,per", [(0, 4, 1000), (0, 120, 37), (7, 10, 64), (7, 150, 1000), (5, 60, 8)])
+def test_emulated_successor_units(emu, oracle, mask, max_ply, per):
+    """The one-lane-per-child program over every legal move of random-play
+    positions (first moves to late boards, every piece), cut into ranges that
+    start inside a root's list and inside a placement cell's rows, against the
+    oracle's successor features."""
+    st, _ = oracle.generate_positions(10, mask, max_ply, 900 + max_ply)
+    st = np.ascontiguousarray(st)
+    mv, n, _, _ = oracle.batch_legal_features_actions(st)
+    mv = np.ascontiguousarray(mv)
+    roots, idx = _all_rows(n)
+    want = oracle.batch_successor_features(st, mv, roots, idx)
+    got = _units(emu, st, mv, roots, idx, per)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def test_emulated_successor_units_any_rows(emu, oracle):
+    """Rows no game reaches -- moves onto or from anywhere, pieces not in hand,
+    a finished game, a board past the pieces of a set, roots and slots out of
+    range, roots in any order -- give what the row-by-row program gives."""
+    rng = np.random.default_rng(5)
+    st, _ = oracle.generate_positions(9, 7, 120, 77)
+    st = np.ascontiguousarray(st)
+    mv, n, _, _ = oracle.batch_legal_features_actions(st)
+    mv = np.ascontiguousarray(mv)
+    st[3, 3415] = 1  # finished
+    st[4, 3396:3404] = 9  # more pieces in hand than a set has
+    h = st[:, 2645:2645 + 529]
+    for i in range(len(st)):  # the last 24 slots of each list: made-up moves
+        occ, free = np.nonzero(h[i])[0], np.nonzero(h[i] == 0)[0]
+        for k in range(232, 256):
+            t = int(rng.integers(0, 4))
+            fr = int(rng.choice(occ if len(occ) and rng.random() < 0.7 else free))
+            near = [c + d for c in occ for d in (-23, -22, -1, 1, 22, 23) if 0 <= c + d < 529 and h[i][c + d] == 0]
+            to = int(rng.choice(near if near and rng.random() < 0.6 else (occ if rng.random() < 0.5 else free)))
+            mv[i, k] = [t, int(rng.integers(1, 9)), fr & 255, fr >> 8, to & 255, to >> 8]
+    roots = np.concatenate([np.repeat(np.arange(len(st)), 24), rng.integers(0, len(st), 60), [-1, len(st), 2, 2]])
+    idx = np.concatenate([np.tile(np.arange(232, 256), len(st)), rng.integers(0, 40, 60), [0, 0, 256, -1]])
+    roots, idx = roots.astype(np.int64), idx.astype(np.int64)
+    idx[: 24 * len(st)] = np.tile(np.arange(232, 256), len(st))
+    want = np.full((len(roots), 122), np.nan, np.float32)
+    emu.emu_successor_rows(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
+                           ctypes.c_int64(st.shape[0]), _p(want))
+    got = _units(emu, st, mv, roots, idx, 50)
+    bad = np.nonzero((got.view(np.uint32) != want.view(np.uint32)).any(1))[0]
+    assert len(bad) == 0, [(int(r), mv[roots[r] % len(st), idx[r] % 256].tolist(),
+                            np.nonzero(got[r] != want[r])[0].tolist()) for r in bad[:6]]
+
+
 @pytest.mark.parametrize("flags,cap", [((1, 1, 1), 0), ((0, 0, 1), 0), ((1, 1, 1), 3)])
 def test_emulated_root_tactical_probe(emu, flags, cap):
     """hive_probe.hpp's group programs, orchestrated as hive_probe.hip's

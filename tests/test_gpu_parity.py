@@ -370,3 +370,26 @@ def test_random_play_pair_counter_scratch(ext):
         assert rc == 0
         torch.cuda.synchronize()
         assert torch.equal(st, want_states) and torch.equal(plies, want_plies)
+
+
+@pytest.mark.parametrize("mask,rows", [(0, 18432), (0, 18433), (7, 18465)])
+def test_successor_rows_both_programs(ext, oracle, mask, rows):
+    """Successor features on both sides of the row count from which a batch's
+    children are worked out one lane each (18,432), rows of whole lists then
+    rows in random order with some out of range, against the oracle."""
+    st, _ = oracle.generate_positions(420, mask, 120, 4100 + mask)
+    mv, n, _, _ = oracle.batch_legal_features_actions(st)
+    roots = np.concatenate([np.full(int(k), i, np.int64) for i, k in enumerate(n)])
+    idx = np.concatenate([np.arange(int(k), dtype=np.int64) for k in n])
+    rng = np.random.default_rng(rows)
+    more = rng.integers(0, len(roots), rows)
+    roots, idx = np.concatenate([roots, roots[more]])[:rows], np.concatenate([idx, idx[more]])[:rows]
+    want = oracle.batch_successor_features(st, mv, roots, idx)
+    bad = rng.integers(0, rows, 40)
+    want[bad] = 0.0
+    roots, idx = roots.copy(), idx.copy()
+    roots[bad[:20]] = len(st)
+    idx[bad[20:]] = -1
+    got = ext.fnn_successor_features_batch(torch.from_numpy(st).cuda(), torch.from_numpy(mv).cuda(),
+                                           torch.from_numpy(roots).cuda(), torch.from_numpy(idx).cuda(), rows)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))

@@ -6,7 +6,7 @@
 // LayerNorm, fc2, value head, action tower over [root | successor]
 // embeddings, scatter into [T, 256] logits, softmax, child-Q scatter.  Here
 // the whole network runs in one kernel per row kind, with the weights held in
-// LDS and the three layer products on fp32 matrix cores:
+// LDS and the three layer products on matrix cores:
 //
 //   k_leaf_mlp<root>   per leaf row: embedding e = fc2(LN(sigmoid(fc1 x))),
 //                      value tanh(value_fc e), and the root half of the
@@ -21,27 +21,40 @@
 //                      priors / child Q (= -child value) as [T][256] rows,
 //                      zero beyond the legal count.
 //
-// Matrix-core layout (v_mfma_f32_16x16x4f32, D = A.B + C, A 16x4, B 4x16):
-// lane l holds A[l%16][l/16], B[l/16][l%16] and D[4(l/16)+i][l%16] in its
-// four accumulator registers i.  A wave evaluates 16 rows at a time and
-// computes every layer transposed, out^T = W . in^T: A = 16 output units of
-// W, B = the inputs of the 16 rows, so after a layer lane l holds, for row
+// The products run on the bf16 matrix cores at float32's accuracy: a float
+// is the exact sum of three bf16 parts (8 significant bits each), and of the
+// nine products of two such sums the six that reach 2^-26 of the whole are
+// taken, v_mfma_f32_16x16x32_bf16 each, accumulated in float32.  That is six
+// times the multiplications at sixteen times the rate of the fp32 matrix
+// instruction; what is left out is a quarter of a float32 rounding.  The
+// weights are split once per evaluation, the activations as they come.
+// Measured against the fp32 instruction (427 K successor rows): 143 -> 91 us,
+// and the outputs' distance from float64 the same (1.4e-7 / 1.4e-7 to 8.5e-7 /
+// 7.7e-7 relative over the seeds tried).  Bound now by the element-wise work
+// (~800 VALU a tile), the matrix pipe and 96 KB of LDS reads a tile, about
+// equal parts.
+//
+// Matrix-core layout (16x16x32, D = A.B + C, A 16x32, B 32x16): lane l holds
+// A[l%16][8 (l/16) + j], B[8 (l/16) + j][l%16] (j < 8) and D[4(l/16)+i][l%16]
+// in its four accumulator registers i.  A wave evaluates 16 rows at a time
+// and computes every layer transposed, out^T = W . in^T: A = 16 output units
+// of W, B = the inputs of the 16 rows, so after a layer lane l holds, for row
 // l%16, the 16 units {16t + 4(l/16) + i : t, i < 4} of its output.  Those are
-// exactly the B operands the next layer needs when the K index of step s for
-// lane group g = l/16 is 16(s/4) + 4g + s%4: no transposes, no LDS traffic
-// between layers.  The weights are stored in LDS pre-permuted to that K
-// order ([step][lane][tile] float4 per lane, conflict-free 16-byte reads).
-// The first layer reads the features in their natural order, K index 32g + s
-// for lane group g (a lane loads 32 consecutive features of its row).
+// exactly the B operands the next layer needs when the input of step s at
+// lane group g = l/16, element j is unit 16 (2s + j/4) + 4g + j%4: no
+// transposes, no LDS traffic between layers.  The weights are stored in LDS
+// pre-permuted to that order ([step][tile][part][lane], conflict-free 16-byte
+// reads).  The first layer reads the features as they lie: step s, lane group
+// g takes features 32 s + 8 g + j.
 //
 // LayerNorm, value and logit reductions over the 64 units of a row are a
 // sum over the lane's 16 units plus two cross-lane steps (lanes l, l^16,
 // l^32, l^48 share a row).
 //
-// Floating point: fp32 throughout with the reference's operations (eps 1e-5,
-// biased variance; sigmoid from the hardware exp2 / reciprocal);
-// summation orders differ from torch's GEMMs, so results agree with the
-// torch composition to ~1e-6 relative, not bit for bit.
+// Floating point: everything between the products in fp32 with the reference's
+// operations (eps 1e-5, biased variance; sigmoid from the hardware exp2 /
+// reciprocal); summation orders differ from torch's GEMMs, so results agree
+// with the torch composition to ~1e-6 relative, not bit for bit.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -53,74 +66,94 @@ namespace {
 constexpr int kE = 64;       // hidden / embedding / action-tower width served here
 constexpr int kFMax = 128;   // feature rows up to 128 wide (Hive FNN: 122)
 constexpr int kSlots = 256;  // legal-slot rows of priors / child Q
-// 8 waves share one LDS copy of the weights: 2 resident blocks (67 KB LDS
-// each) per CU give 4 waves per SIMD to overlap the element-wise work and
-// loads with the matrix cores
-constexpr int kBlockWaves = 8;
-constexpr int kMaxBlocks = 512;  // 2 resident blocks on each of 256 CUs
+// 16 waves share one LDS copy of the split weights (98 KB): one resident block
+// per CU, 4 waves per SIMD to overlap the element-wise work and loads with
+// the matrix cores
+constexpr int kBlockWaves = 16;
+constexpr int kMaxBlocks = 256;  // one resident block on each of 256 CUs
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
+// The network in the order the MLP kernels keep it in LDS, split into bf16
+// parts once per evaluation (pack_net_at, in the evaluation's first launch),
+// so that each of their blocks fills LDS with straight 16-byte copies.
+// Element [step][tile][part][lane] holds the lane's eight weights.
+struct PackedNet {
+    b8 w1[4][4][3][64];     // fc1, input 32 s + 8 g + j
+    b8 w2[2][4][3][64];     // fc2, input 16 (2s + j/4) + 4g + j%4
+    b8 w3[2][2][4][3][64];  // action_fc1: root half, successor half, as fc2
+    float vec[7][kE];
+};
 struct MlpLds {
-    f4 w1[32][64];  // fc1, step s = K index 32g + s
-    f4 w2[16][64];  // fc2, step s = K index 16(s/4) + 4g + s%4
-    f4 w3[16][64];  // action_fc1 root half (root rows) or successor half (successor rows)
+    b8 w1[4][4][3][64];
+    b8 w2[2][4][3][64];
+    b8 w3[2][4][3][64];  // action_fc1 root half (root rows) or successor half (successor rows)
     float vec[7][kE];
 };
 enum { kB1, kLnW, kLnB, kB2, kWv, kWa2, kBa1 };
 
-// The network laid out once per evaluation in the order the MLP kernels keep
-// in LDS (pack_net_at, in the evaluation's first launch), so that each of
-// their blocks fills LDS with straight 16-byte copies instead of gathering
-// and permuting the weights itself.
-struct PackedNet {
-    f4 w1[32][64];
-    f4 w2[16][64];
-    f4 w3[2][16][64];  // action_fc1: root half, successor half
-    float vec[7][kE];
-};
-
-// element i of a [step][lane][tile] array: unit m = 16 tile + lane % 16 and the
-// step / lane group dependent K index (fc1: 32 g + s; the 64-wide layers:
-// 16 (s / 4) + 4 g + s % 4)
-__device__ __forceinline__ void perm_index(int i, bool first, int& m, int& k) {
-    const int t = i & 3, l = (i >> 2) & 63, s = i >> 8;
-    m = 16 * t + (l & 15);
-    k = first ? 32 * (l >> 4) + s : 16 * (s >> 2) + 4 * (l >> 4) + (s & 3);
+// x as three bf16 parts, x = p0 + p1 + p2 exactly (each remainder is exact in
+// float32 and has eight bits fewer; parts below bf16's range are dropped)
+__device__ __forceinline__ void split3(f2 x, b2& p0, b2& p1, b2& p2) {
+    p0 = __builtin_convertvector(x, b2);
+    const f2 r = x - __builtin_convertvector(p0, f2);
+    p1 = __builtin_convertvector(r, b2);
+    p2 = __builtin_convertvector(r - __builtin_convertvector(p1, f2), b2);
 }
 
-// thread i of the packing writes float i of the packed layout (k_leaf_prep's
+constexpr float kSplitMost = 3.38e38f;  // the largest bf16 is 3.39e38
+
+// Weight i of a [step][tile][lane][j] array: unit m = 16 tile + lane % 16 and
+// its input k; at: the element's place in the split array, parts 64 * 8 apart.
+__device__ __forceinline__ void perm_index(int i, bool first, int& m, int& k, int& at) {
+    const int j = i & 7, l = (i >> 3) & 63, t = (i >> 9) & 3, s = i >> 11, g = l >> 4;
+    m = 16 * t + (l & 15);
+    k = first ? 32 * s + 8 * g + j : 16 * (2 * s + (j >> 2)) + 4 * g + (j & 3);
+    at = ((s * 4 + t) * 3 * 64 + l) * 8 + j;
+}
+__device__ __forceinline__ void put_split(__bf16* dst, int at, float w) {
+    b2 p0, p1, p2;
+    split3(f2{w, 0.0f}, p0, p1, p2);
+    dst[at] = p0[0];
+    dst[at + 512] = p1[0];
+    dst[at + 1024] = p2[0];
+}
+
+// thread i of the packing splits weight i of the packed layout (k_leaf_prep's
 // packing blocks)
+constexpr int kPack1 = 4 * 4 * 64 * 8, kPack2 = 2 * 4 * 64 * 8;
 __device__ __forceinline__ void pack_net_at(int i, const float* __restrict__ w1, int F, const float* __restrict__ b1,
                                             const float* __restrict__ lnw, const float* __restrict__ lnb,
-                                            const float* __restrict__ w2, const float* __restrict__ b2,
+                                            const float* __restrict__ w2, const float* __restrict__ b2_,
                                             const float* __restrict__ wv, const float* __restrict__ a1w,
                                             const float* __restrict__ a1b, const float* __restrict__ a2w,
                                             PackedNet* __restrict__ out) {
-    constexpr int n1 = 32 * 64 * 4, n2 = 16 * 64 * 4;
-    int m, k;
-    if (i < n1) {
-        perm_index(i, true, m, k);
-        reinterpret_cast<float*>(&out->w1[0][0])[i] = k < F ? w1[m * F + k] : 0.0f;
-    } else if (i < n1 + n2) {
-        perm_index(i - n1, false, m, k);
-        reinterpret_cast<float*>(&out->w2[0][0])[i - n1] = w2[m * kE + k];
-    } else if (i < n1 + 3 * n2) {
-        const int j = i - n1 - n2, half = j / n2;
-        perm_index(j - half * n2, false, m, k);
-        reinterpret_cast<float*>(&out->w3[0][0][0])[j] = a1w[m * 2 * kE + half * kE + k];
-    } else if (i < n1 + 3 * n2 + kE) {
-        const int u = i - n1 - 3 * n2;
+    int m, k, at;
+    if (i < kPack1) {
+        perm_index(i, true, m, k, at);
+        put_split(reinterpret_cast<__bf16*>(&out->w1), at, k < F ? w1[m * F + k] : 0.0f);
+    } else if (i < kPack1 + kPack2) {
+        perm_index(i - kPack1, false, m, k, at);
+        put_split(reinterpret_cast<__bf16*>(&out->w2), at, w2[m * kE + k]);
+    } else if (i < kPack1 + 3 * kPack2) {
+        const int j = i - kPack1 - kPack2, half = j / kPack2;
+        perm_index(j - half * kPack2, false, m, k, at);
+        put_split(reinterpret_cast<__bf16*>(&out->w3[half]), at, a1w[m * 2 * kE + half * kE + k]);
+    } else if (i < kPack1 + 3 * kPack2 + kE) {
+        const int u = i - kPack1 - 3 * kPack2;
         out->vec[kB1][u] = b1[u];
         out->vec[kLnW][u] = lnw[u];
         out->vec[kLnB][u] = lnb[u];
-        out->vec[kB2][u] = b2[u];
+        out->vec[kB2][u] = b2_[u];
         out->vec[kWv][u] = wv[u];
         out->vec[kWa2][u] = a2w[u];
         out->vec[kBa1][u] = a1b[u];
     }
 }
-constexpr int kPackThreads = 32 * 64 * 4 + 3 * 16 * 64 * 4 + kE;
+constexpr int kPackThreads = kPack1 + 3 * kPack2 + kE;
 constexpr int kPackBlocks = (kPackThreads + 255) / 256;
 
 // The first launch of a fused leaf evaluation, three kinds of 256-thread
@@ -196,8 +229,28 @@ __device__ __forceinline__ float row_sum(float v) {
     return v;
 }
 
-__device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+// c + a . b over 32 inputs of float32 operands in three parts (see above);
+// the smallest products first
+__device__ __forceinline__ f4 mfma3(const b8 (&a)[3][64], int lane, const b8 (&b)[3], f4 c) {
+    const b8 a0 = a[0][lane], a1 = a[1][lane], a2 = a[2][lane];
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[2], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[1], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[0], c, 0, 0, 0);
+}
+// eight inputs x(0) .. x(7) as the three parts of a B operand
+template <typename Fn>
+__device__ __forceinline__ void split8(Fn x, b8 (&b)[3]) {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+        b2 p0, p1, p2;
+        split3(f2{x(j), x(j + 1)}, p0, p1, p2);
+        b[0][j] = p0[0], b[0][j + 1] = p0[1];
+        b[1][j] = p1[0], b[1][j + 1] = p1[1];
+        b[2][j] = p2[0], b[2][j + 1] = p2[1];
+    }
 }
 
 __device__ __forceinline__ f4 vec4(const MlpLds& L, int which, int t, int g) {
@@ -227,36 +280,39 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
     // with no tile leaves before filling LDS
     if ((int64_t)blockIdx.x >= ntiles) return;
     if (pk) {  // the packed layout: straight 16-byte copies, every load issued before the first store
-        constexpr int kT = 64 * kBlockWaves, k12 = 48 * 64 / kT, k3 = 16 * 64 / kT;
-        static_assert(48 * 64 % kT == 0 && 16 * 64 % kT == 0 && 7 * kE / 4 <= kT, "whole copy rounds");
+        constexpr int kT = 64 * kBlockWaves, k12 = (sizeof(L.w1) + sizeof(L.w2)) / 16, k3 = sizeof(L.w3) / 16;
+        constexpr int n12 = (k12 + kT - 1) / kT, n3 = (k3 + kT - 1) / kT;
+        static_assert(7 * kE / 4 <= kT && sizeof(L.w1) % 16 == 0, "16-byte copies");
         const int tid = threadIdx.x;
-        const f4* src = &pk->w1[0][0];
-        const f4* s3 = &pk->w3[kRoot ? 0 : 1][0][0];
-        f4 c12[k12], c3[k3], cv = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        const f4* src = reinterpret_cast<const f4*>(&pk->w1);
+        const f4* s3 = reinterpret_cast<const f4*>(&pk->w3[kRoot ? 0 : 1]);
+        f4 c12[n12], c3[n3], cv = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int k = 0; k < k12; k++) c12[k] = src[tid + k * kT];  // w1, w2
+        for (int k = 0; k < n12; k++)
+            if (tid + k * kT < k12) c12[k] = src[tid + k * kT];  // w1, w2
 #pragma unroll
-        for (int k = 0; k < k3; k++) c3[k] = s3[tid + k * kT];
+        for (int k = 0; k < n3; k++)
+            if (tid + k * kT < k3) c3[k] = s3[tid + k * kT];
         if (tid < 7 * kE / 4) cv = reinterpret_cast<const f4*>(&pk->vec[0][0])[tid];
-        f4* dst = &L.w1[0][0];
+        f4* dst = reinterpret_cast<f4*>(&L.w1);
+        f4* d3 = reinterpret_cast<f4*>(&L.w3);
 #pragma unroll
-        for (int k = 0; k < k12; k++) dst[tid + k * kT] = c12[k];
+        for (int k = 0; k < n12; k++)
+            if (tid + k * kT < k12) dst[tid + k * kT] = c12[k];
 #pragma unroll
-        for (int k = 0; k < k3; k++) (&L.w3[0][0])[tid + k * kT] = c3[k];
+        for (int k = 0; k < n3; k++)
+            if (tid + k * kT < k3) d3[tid + k * kT] = c3[k];
         if (tid < 7 * kE / 4) reinterpret_cast<f4*>(&L.vec[0][0])[tid] = cv;
-    } else {  // permuted weights gathered into LDS (perm_index)
-        int m, k;
-        float* l1 = reinterpret_cast<float*>(&L.w1[0][0]);
-        for (int i = threadIdx.x; i < 32 * 64 * 4; i += blockDim.x) {
-            perm_index(i, true, m, k);
-            l1[i] = k < F ? w1[m * F + k] : 0.0f;
+    } else {  // weights gathered, permuted and split into LDS (perm_index)
+        int m, k, at;
+        for (int i = threadIdx.x; i < kPack1; i += blockDim.x) {
+            perm_index(i, true, m, k, at);
+            put_split(reinterpret_cast<__bf16*>(&L.w1), at, k < F ? w1[m * F + k] : 0.0f);
         }
-        float* l2 = reinterpret_cast<float*>(&L.w2[0][0]);
-        float* l3 = reinterpret_cast<float*>(&L.w3[0][0]);
-        for (int i = threadIdx.x; i < 16 * 64 * 4; i += blockDim.x) {
-            perm_index(i, false, m, k);
-            l2[i] = w2[m * kE + k];
-            l3[i] = a1w[m * 2 * kE + (kRoot ? 0 : kE) + k];
+        for (int i = threadIdx.x; i < kPack2; i += blockDim.x) {
+            perm_index(i, false, m, k, at);
+            put_split(reinterpret_cast<__bf16*>(&L.w2), at, w2[m * kE + k]);
+            put_split(reinterpret_cast<__bf16*>(&L.w3), at, a1w[m * 2 * kE + (kRoot ? 0 : kE) + k]);
         }
         if (threadIdx.x < kE) {
             const int u = threadIdx.x;
@@ -275,7 +331,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
     for (int64_t tile = (int64_t)blockIdx.x + (int64_t)gridDim.x * (threadIdx.x >> 6); tile < ntiles;
          tile += (int64_t)gridDim.x * kBlockWaves) {
         // the weights are re-read from LDS in every tile: hoisted out of the
-        // loop they would take ~400 registers and leave one wave per SIMD
+        // loop they would take hundreds of registers and leave one wave per SIMD
         __asm__ volatile("" ::: "memory");
         const int64_t row = tile * 16 + (lane & 15);
         const bool ok = row < rows;
@@ -287,13 +343,14 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 #pragma unroll
             for (int t = 0; t < 4; t++) rh[t] = *reinterpret_cast<const f4*>(R + leaf * kE + 16 * t + 4 * g);
         }
-        // features 32g .. 32g+31 of this lane's row
+        // features 32 s + 8 g + j of this lane's row
         float x[32];
-        const float* xr = X + (ok ? row : 0) * F + 32 * g;
+        const float* xr = X + (ok ? row : 0) * F + 8 * g;
 #pragma unroll
         for (int p = 0; p < 16; p++) {
+            const int at = 32 * (p >> 2) + 2 * (p & 3);
             float2 v = make_float2(0.0f, 0.0f);
-            if (ok && 32 * g + 2 * p < F) v = *reinterpret_cast<const float2*>(xr + 2 * p);
+            if (ok && 8 * g + at < F) v = *reinterpret_cast<const float2*>(xr + at);
             x[2 * p] = v.x;
             x[2 * p + 1] = v.y;
         }
@@ -301,13 +358,27 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
         f4 acc[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        // a feature past the parts' range (infinite, or rounding to it) has no
+        // split: its tile's first layer is summed plainly
+        float most = 0.0f;
 #pragma unroll
-        for (int s = 0; s < 32; s++) {
-            const f4 a = L.w1[s][lane];
-            acc[0] = mfma(a.x, x[s], acc[0]);
-            acc[1] = mfma(a.y, x[s], acc[1]);
-            acc[2] = mfma(a.z, x[s], acc[2]);
-            acc[3] = mfma(a.w, x[s], acc[3]);
+        for (int j = 0; j < 32; j += 2) most = fmaxf(fmaxf(most, fabsf(x[j])), fabsf(x[j + 1]));
+        if (__ballot(most > kSplitMost)) {
+            for (int k = 0; k < F; k++) {
+                const float xk = ok ? X[row * F + k] : 0.0f;
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[t][i] += w1[(16 * t + 4 * g + i) * F + k] * xk;
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                b8 b[3];
+                split8([&](int j) { return x[8 * s + j]; }, b);
+#pragma unroll
+                for (int t = 0; t < 4; t++) acc[t] = mfma3(L.w1[s][t], lane, b, acc[t]);
+            }
         }
         // sigmoid + LayerNorm over the row's 64 units
         float sum = 0.0f;
@@ -341,13 +412,11 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 #pragma unroll
         for (int t = 0; t < 4; t++) e[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int s = 0; s < 16; s++) {
-            const f4 a = L.w2[s][lane];
-            const float b = acc[s >> 2][s & 3];
-            e[0] = mfma(a.x, b, e[0]);
-            e[1] = mfma(a.y, b, e[1]);
-            e[2] = mfma(a.z, b, e[2]);
-            e[3] = mfma(a.w, b, e[3]);
+        for (int s = 0; s < 2; s++) {
+            b8 b[3];
+            split8([&](int j) { return acc[2 * s + (j >> 2)][j & 3]; }, b);
+#pragma unroll
+            for (int t = 0; t < 4; t++) e[t] = mfma3(L.w2[s][t], lane, b, e[t]);
         }
         float v = 0.0f;
 #pragma unroll
@@ -365,13 +434,11 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 #pragma unroll
         for (int t = 0; t < 4; t++) h[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int s = 0; s < 16; s++) {
-            const f4 a = L.w3[s][lane];
-            const float b = e[s >> 2][s & 3];
-            h[0] = mfma(a.x, b, h[0]);
-            h[1] = mfma(a.y, b, h[1]);
-            h[2] = mfma(a.z, b, h[2]);
-            h[3] = mfma(a.w, b, h[3]);
+        for (int s = 0; s < 2; s++) {
+            b8 b[3];
+            split8([&](int j) { return e[2 * s + (j >> 2)][j & 3]; }, b);
+#pragma unroll
+            for (int t = 0; t < 4; t++) h[t] = mfma3(L.w3[s][t], lane, b, h[t]);
         }
         if constexpr (kRoot) {
             if (ok) {

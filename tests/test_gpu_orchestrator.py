@@ -731,3 +731,36 @@ def test_reserve_candidates_match_oracle(mask, max_ply, immobile):
         c2 = ext.candidate_rows(torch.from_numpy(want_q).cuda(), torch.from_numpy(valid).cuda(),
                                 torch.from_numpy(pri).cuda(), 16, 6)
         assert np.array_equal(_np(c2), want_c)
+
+
+@pytest.mark.parametrize("T,each,scale", [(1, 1, 1.0), (3, 5, 1e-3), (17, 16, 1.0), (40, 33, 1e4)])
+def test_leaf_eval_products_against_float64(T, each, scale):
+    """The network's products (float32 operands in three bf16 parts) at tile
+    edges and remainders, features from small to large and infinite or NaN
+    ones among them, against float64: the values and child Q of finite rows
+    within 1e-5 (64 to 122 float32 terms a sum, sigmoids in between), and the
+    rows of non-finite features non-finite where float64's are."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(21)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    N = T * each
+    f = (torch.rand((T + N, 122), generator=g, device="cuda") - 0.3) * scale
+    f[:, ::3] = torch.round(f[:, ::3])
+    odd = [r for r in (0, T + N // 2, T + N - 1) if T + N > 3]
+    for r, v in zip(odd, (float("inf"), float("-inf"), float("nan"))):
+        f[r, 7 + r % 100] = v
+    n = torch.full((T,), each, dtype=torch.int32, device="cuda")
+    off = torch.arange(T, device="cuda", dtype=torch.int64) * each
+    leaf = torch.arange(T, device="cuda").repeat_interleave(each)
+    _, value, child_q = ext.fnn_leaf_eval(f, T, off, n, leaf, net)
+    net64 = seeded_large(21).double()
+    with torch.no_grad():
+        want = net64.value_head(net64.encode(f.double())).squeeze(1)
+    got = torch.cat([value, -child_q[:, :each].reshape(-1)]).double()
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    ok = torch.isfinite(want)
+    assert float((got[ok] - want[ok]).abs().max()) < 1e-5

@@ -197,6 +197,12 @@ def _select_outputs(T: int, whole_rows: bool = False):
     vlen = new((T,), dtype=torch.int32, device="cuda")
     return leaf, paths, plen, vl, vlen
 
+# fused lists of more positions than this are taken in turn order: up to here the
+# device holds nearly every position at once, and the order costs a launch
+# (ordered / index order, us: 1 position 25 / 22, 4,096 37 / 32, 8,192 42 / 39,
+# 12,288 55 / 59; with every piece 8,192 104 / 98, 12,288 113 / 125)
+_order_min_batch = 10240
+
 _lib = None
 _lib_lock = threading.Lock()
 # root_tactical_probe_batch_noalloc: per device, an event recorded after the
@@ -325,9 +331,9 @@ class HiveGpuExtension:
     def generate_legal_moves_features_actions_batch(self, states: torch.Tensor, batch_size: int,
                                                     ordered: bool = True):
         """Fused: (moves, num_legal, features, action_indices) in one pass.  With
-        `ordered` (default) the positions are taken in buckets of turns, latest
-        first (hg_legal_features_actions_ordered): the same outputs, a shorter
-        launch on batches of mixed game stages.  Its int32 workspace is kept per
+        `ordered` (default) the positions of a large batch are taken in buckets of
+        turns, latest first (hg_legal_features_actions_ordered): the same
+        outputs, a shorter launch on batches of mixed game stages.  Its int32 workspace is kept per
         (device, stream) and its two count arrays are used in turn, so a call
         made while the stream is being captured into a HIP graph (whose replays
         would all repeat the captured turn) takes the index order instead."""
@@ -337,7 +343,7 @@ class HiveGpuExtension:
         n = torch.empty((B,), dtype=torch.int32, device="cuda")
         feat = torch.empty((B, FNN_FEAT_DIM), dtype=torch.float32, device="cuda")
         act = torch.empty((B, MAX_LEGAL_MOVES), dtype=torch.int32, device="cuda")
-        if ordered and B > 0 and not torch.cuda.is_current_stream_capturing():
+        if ordered and B > _order_min_batch and not torch.cuda.is_current_stream_capturing():
             stream = _stream()
             key = (torch.cuda.current_device(), stream)
             need = int(self._lib.hg_legal_features_actions_ordered_workspace(B)) // 4

@@ -867,20 +867,28 @@ int hg_compute_centroids(const uint8_t* states, int64_t B, int32_t* centroids, v
 
 int64_t hg_successor_rows_workspace(int64_t T) { return T <= 0 ? 0 : 8 * (T + 1 + 2 * T * (int64_t)kMaxLegal); }
 
-int hg_successor_rows(const uint8_t* states, const uint8_t* legal_moves, const int32_t* num_legal, int64_t T,
-                      void* workspace, float* features, void* stream) {
+int hg_successor_plan(const int32_t* num_legal, int64_t T, void* workspace, void* stream) {
     if (T <= 0) return 0;
     if (((uintptr_t)workspace & 7)) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
-    if (T <= kPlanLeaves) {
-        const RowsPlan R = rows_plan_of(workspace, T);
-        hipLaunchKernelGGL(k_rows_plan, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, num_legal, T, R.offsets,
-                           R.total, R.a2r, R.mi);
-    } else {
-        int e = successor_rows_plan_large(num_legal, T, workspace, s);
-        if (e) return e;
-    }
-    return successor_rows_after_plan(states, legal_moves, T, workspace, features, s);
+    if (T > kPlanLeaves) return successor_rows_plan_large(num_legal, T, workspace, s);
+    const RowsPlan R = rows_plan_of(workspace, T);
+    hipLaunchKernelGGL(k_rows_plan, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, s, num_legal, T, R.offsets,
+                       R.total, R.a2r, R.mi);
+    return finish();
+}
+
+int hg_successor_planned_rows(const uint8_t* states, const uint8_t* legal_moves, int64_t T, void* workspace,
+                              float* features, void* stream) {
+    if (T <= 0) return 0;
+    if (((uintptr_t)workspace & 7)) return (int)hipErrorInvalidValue;
+    return successor_rows_after_plan(states, legal_moves, T, workspace, features, (hipStream_t)stream);
+}
+
+int hg_successor_rows(const uint8_t* states, const uint8_t* legal_moves, const int32_t* num_legal, int64_t T,
+                      void* workspace, float* features, void* stream) {
+    const int e = hg_successor_plan(num_legal, T, workspace, stream);
+    return e ? e : hg_successor_planned_rows(states, legal_moves, T, workspace, features, stream);
 }
 
 int hg_fnn_successor_features(const uint8_t* states, const uint8_t* legal_moves, int64_t num_roots,

@@ -70,6 +70,8 @@ _SIGS = {
     "hg_compute_centroids": [_c_void_p, _c_i64, _c_void_p, _c_void_p],
     "hg_fnn_successor_features": [_c_void_p, _c_void_p, _c_i64, _c_void_p, _c_void_p, _c_i64, _c_void_p,
                                   _c_void_p],
+    "hg_successor_plan": [_c_void_p, _c_i64, _c_void_p, _c_void_p],
+    "hg_successor_planned_rows": [_c_void_p, _c_void_p, _c_i64, _c_void_p, _c_void_p, _c_void_p],
     "hg_queen_escape_flags": [_c_void_p, _c_i64, _c_void_p, _c_void_p],
     "hg_fnn_leaf_eval": [_c_void_p, _c_i64, _c_i64, ctypes.c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                          _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, ctypes.c_float,
@@ -410,6 +412,23 @@ class HiveGpuExtension:
                                                    action_to_root.data_ptr(), move_indices.data_ptr(), N,
                                                    feat.data_ptr(), _stream()), "fnn_successor_features_batch")
         return feat
+
+    def fnn_list_successor_features_batch(self, states, legal_moves, num_legal, batch_size: int):
+        """Every legal successor of `batch_size` roots (extension): (features
+        [N, 122] f32, action_to_root [N] int64), rows in (root, slot) order,
+        the row map made on the device; one host read (N)."""
+        B = int(batch_size)
+        states = _state_rows(states, B)
+        legal_moves = _dev(legal_moves, "legal_moves", torch.uint8, (MAX_LEGAL_MOVES, SIZEOF_GPU_MOVE), B)
+        num_legal = _dev(num_legal, "num_legal", torch.int32, (), B)
+        ws = torch.empty((max(1, int(self._lib.hg_successor_rows_workspace(B)) // 8),), dtype=torch.int64, device="cuda")
+        _check(self._lib.hg_successor_plan(num_legal.data_ptr(), B, ws.data_ptr(), _stream()), "successor_plan")
+        N = int(ws[B].item()) if B > 0 else 0
+        feat = torch.empty((N, FNN_FEAT_DIM), dtype=torch.float32, device="cuda")
+        if N > 0:
+            _check(self._lib.hg_successor_planned_rows(states.data_ptr(), legal_moves.data_ptr(), B, ws.data_ptr(),
+                                                       feat.data_ptr(), _stream()), "successor_planned_rows")
+        return feat, ws[B + 1: B + 1 + N]
 
     # ---- fused FNN leaf evaluation (no reference counterpart; see include/hive_gpu.h)
     def fnn_leaf_eval(self, features, T: int, offsets, num_legal, succ_leaf, net, head_biases=None):

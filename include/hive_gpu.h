@@ -200,6 +200,12 @@ int hg_legal_mask(const uint8_t* states, int64_t B, uint8_t* moves, int32_t* num
 int64_t hg_successor_rows_workspace(int64_t T);
 int hg_successor_rows(const uint8_t* states, const uint8_t* legal_moves, const int32_t* num_legal, int64_t T,
                       void* workspace, float* features, void* stream);
+/* hg_successor_rows in its two steps, for a caller that sizes the features by
+ * the total between them: the plan (offsets, total, map into the workspace),
+ * then the planned rows' features (`total` rows of 122). */
+int hg_successor_plan(const int32_t* num_legal, int64_t T, void* workspace, void* stream);
+int hg_successor_planned_rows(const uint8_t* states, const uint8_t* legal_moves, int64_t T, void* workspace,
+                              float* features, void* stream);
 
 /* hg_fnn_leaf_eval over the leaves' own legal lists, with no host
  * synchronisation: hg_successor_rows into the workspace, then the network

@@ -200,12 +200,6 @@ constexpr int64_t kSuccGrid = 256 * 16;
 constexpr int kSuccWaves = 4;
 // rows per block: a kSuccSpread-th of the batch, from kSuccShort to kSuccBlock
 constexpr int kSuccShort = 8, kSuccBlock = 32, kSuccSpread = 2048;
-// Batches of at most kSuccStream rows go row by row, a lane group each
-// (successor_row): one row takes about a third of a pass's time.  Leaf
-// evaluation by rows / by passes, us: mid-game base game 14 K rows 65 / 73,
-// 27 K 88 / 76, 53 K 133 / 94; every piece 9 K rows 77 / 96, 19 K 104 / 102,
-// 38 K 155 / 110; after two plies 15 K 61 / 60, 31 K 73 / 61
-constexpr int kSuccStream = 18432;
 // lane groups a batch of leaves is spread over by cutting its lists into parts
 constexpr int kSuccParts = 8, kSuccTarget = 8192;
 
@@ -266,7 +260,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))
         for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < blocks; p += groups) {
             range(p, lo, hi);
             general |= successor_range<Ix>(GS[grp], K, states, legal, MapRows{a2r, midx}, lo, hi, num_roots, kZeroRow,
-                                           lane, feat_out);
+                                           lane, FeatureRows{feat_out});
         }
         __syncthreads();  // the marks, read by other lanes
         marks = hw_wave_any(general);
@@ -695,10 +689,11 @@ __global__ __launch_bounds__(256) void k_rows_plan(const int32_t* __restrict__ n
 // work enough to hide a pass's latency; with many after one window's rows --
 // the launch ends with its longest waves, and the lists that need a second
 // window (a fifth of the mid-game ones) are other lane groups' work.
-template <typename Ix>
+template <typename Ix, class Out>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))) void k_successor_rows(
     const uint8_t* __restrict__ states, const uint8_t* __restrict__ legal, const int64_t* __restrict__ a2r,
-    const int64_t* __restrict__ midx, const int64_t* __restrict__ offsets, int64_t T, float* feat_out) {
+    const int64_t* __restrict__ midx, const int64_t* __restrict__ offsets, int64_t T, Out out) {
+    float* const feat_out = out.feat;
     __shared__ SuccBoard GS[kPosPerWave];
     __shared__ SuccTables K;
     const int lane = threadIdx.x, grp = lane >> 5;
@@ -737,7 +732,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))
             if (!hw_wave_any(lo < hi)) continue;
             if (!ready) load_succ_tables(K);
             ready = true;
-            general |= successor_range<Ix>(GS[grp], K, states, legal, src, lo, hi, T, kZeroRow, lane, feat_out);
+            general |= successor_range<Ix>(GS[grp], K, states, legal, src, lo, hi, T, kZeroRow, lane, out);
         }
         __syncthreads();  // the marks, read by other lanes
         marks = hw_wave_any(general);
@@ -975,7 +970,7 @@ int successor_rows_plan_large(const int32_t* num_legal, int64_t T, void* workspa
 }
 
 int successor_rows_after_plan(const uint8_t* states, const uint8_t* legal_moves, int64_t T, void* workspace,
-                              float* features, hipStream_t s) {
+                              float* features, hipStream_t s, UnitRecord* units, uint32_t* info) {
     const RowsPlan R = rows_plan_of(workspace, T);
     // every part of every leaf, and for a small batch a lane group per row (at
     // most 256 a leaf); workgroups with nothing to do end at once
@@ -983,12 +978,19 @@ int successor_rows_after_plan(const uint8_t* states, const uint8_t* legal_moves,
     const int64_t streams = T * kMaxLegal / kPosPerWave < kSuccGrid ? T * kMaxLegal / kPosPerWave : kSuccGrid;
     pairs = pairs < streams ? streams : pairs;
     const unsigned grid = (unsigned)(pairs < 16 * kSuccGrid ? pairs : 16 * kSuccGrid);
-    if (successor_narrow(T * kMaxLegal, T))  // at most 256 rows per leaf
-        hipLaunchKernelGGL(k_successor_rows<uint32_t>, dim3(grid), dim3(64), 0, s, states, legal_moves, R.a2r, R.mi,
-                           R.offsets, T, features);
-    else
-        hipLaunchKernelGGL(k_successor_rows<int64_t>, dim3(grid), dim3(64), 0, s, states, legal_moves, R.a2r, R.mi,
-                           R.offsets, T, features);
+    const bool narrow = successor_narrow(T * kMaxLegal, T);  // at most 256 rows per leaf
+    auto launch = [&](auto kernel, auto out) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, states, legal_moves, R.a2r, R.mi, R.offsets, T, out);
+    };
+    if (units) {
+        const UnitRows out{features, units, info};
+        if (narrow) launch(k_successor_rows<uint32_t, UnitRows>, out);
+        else launch(k_successor_rows<int64_t, UnitRows>, out);
+    } else {
+        const FeatureRows out{features};
+        if (narrow) launch(k_successor_rows<uint32_t, FeatureRows>, out);
+        else launch(k_successor_rows<int64_t, FeatureRows>, out);
+    }
     return finish();
 }
 

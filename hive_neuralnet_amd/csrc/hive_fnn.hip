@@ -44,8 +44,11 @@
 // lane group g = l/16, element j is unit 16 (2s + j/4) + 4g + j%4: no
 // transposes, no LDS traffic between layers.  The weights are stored in LDS
 // pre-permuted to that order ([step][tile][part][lane], conflict-free 16-byte
-// reads).  The first layer reads the features as they lie: step s, lane group
-// g takes features 32 s + 8 g + j.
+// reads).  The first layer's input of step s, lane group g, element j follows
+// the features' six sections of 16 classes: a quarter of each section per lane
+// group (feature_of), so that a lane can build its 32 inputs from a successor's
+// packed record (unit_slice) with the same code in every lane; the counts among
+// them (steps 0 and 2) are one bf16 part exactly.
 //
 // LayerNorm, value and logit reductions over the 64 units of a row are a
 // sum over the lane's 16 units plus two cross-lane steps (lanes l, l^16,
@@ -82,7 +85,7 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 // so that each of their blocks fills LDS with straight 16-byte copies.
 // Element [step][tile][part][lane] holds the lane's eight weights.
 struct PackedNet {
-    b8 w1[4][4][3][64];     // fc1, input 32 s + 8 g + j
+    b8 w1[4][4][3][64];     // fc1, input feature_of(s, g, j)
     b8 w2[2][4][3][64];     // fc2, input 16 (2s + j/4) + 4g + j%4
     b8 w3[2][2][4][3][64];  // action_fc1: root half, successor half, as fc2
     float vec[7][kE];
@@ -106,12 +109,20 @@ __device__ __forceinline__ void split3(f2 x, b2& p0, b2& p1, b2& p2) {
 
 constexpr float kSplitMost = 3.38e38f;  // the largest bf16 is 3.39e38
 
+// The feature that fc1's step s takes at lane group g, element j: sections 0
+// and 2, 1 and 3, 4 and 5 (top pieces, next to the queen; hands, distances;
+// can move, pinned), four classes of each, then eight of the last 32.
+__host__ __device__ constexpr int feature_section(int s, int j) { return s == 2 ? 4 + (j >> 2) : s + 2 * (j >> 2); }
+__host__ __device__ constexpr int feature_of(int s, int g, int j) {
+    return s < 3 ? 16 * feature_section(s, j) + 4 * g + (j & 3) : 96 + 8 * g + j;
+}
+
 // Weight i of a [step][tile][lane][j] array: unit m = 16 tile + lane % 16 and
 // its input k; at: the element's place in the split array, parts 64 * 8 apart.
 __device__ __forceinline__ void perm_index(int i, bool first, int& m, int& k, int& at) {
     const int j = i & 7, l = (i >> 3) & 63, t = (i >> 9) & 3, s = i >> 11, g = l >> 4;
     m = 16 * t + (l & 15);
-    k = first ? 32 * s + 8 * g + j : 16 * (2 * s + (j >> 2)) + 4 * g + (j & 3);
+    k = first ? feature_of(s, g, j) : 16 * (2 * s + (j >> 2)) + 4 * g + (j & 3);
     at = ((s * 4 + t) * 3 * 64 + l) * 8 + j;
 }
 __device__ __forceinline__ void put_split(__bf16* dst, int at, float w) {
@@ -240,6 +251,13 @@ __device__ __forceinline__ f4 mfma3(const b8 (&a)[3][64], int lane, const b8 (&b
     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[1], c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[0], c, 0, 0, 0);
 }
+// the same for inputs that are one bf16 part exactly
+__device__ __forceinline__ f4 mfma3_whole(const b8 (&a)[3][64], int lane, const b8& b, f4 c) {
+    const b8 a0 = a[0][lane], a1 = a[1][lane], a2 = a[2][lane];
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b, c, 0, 0, 0);
+}
 // eight inputs x(0) .. x(7) as the three parts of a B operand
 template <typename Fn>
 __device__ __forceinline__ void split8(Fn x, b8 (&b)[3]) {
@@ -260,7 +278,9 @@ __device__ __forceinline__ f4 vec4(const MlpLds& L, int which, int t, int g) {
 // X: [rows][F] features (F even, <= 128, 8-byte aligned rows).
 // kRoot: R[rows][64] <- Wr e + b_a1, value[rows] <- tanh(wv . e + bv).
 // !kRoot: row -> leaf = succ_leaf[row]; value[rows] <- tanh(wv . e + bv),
-//         logit[rows] <- wa2 . sigmoid(Ws e + R[leaf]) + ba2.
+//         logit[rows] <- wa2 . sigmoid(Ws e + R[leaf]) + ba2; with `units`
+//         and more than kSuccStream rows the features come from the rows' unit
+//         records (X holds the rows marked kRowGeneral only).
 template <bool kRoot>
 __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __restrict__ X, int64_t rows, int F,
                                                   const int64_t* __restrict__ succ_leaf, int64_t T,
@@ -271,7 +291,9 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
                                                   const float* __restrict__ a1b, const float* __restrict__ a2w, float ba2,
                                                   float* __restrict__ R, float* __restrict__ value,
                                                   float* __restrict__ logit, const int64_t* __restrict__ rows_dev,
-                                                  const PackedNet* __restrict__ pk) {
+                                                  const PackedNet* __restrict__ pk,
+                                                  const hw::UnitRecord* __restrict__ units = nullptr,
+                                                  const uint32_t* __restrict__ info = nullptr) {
     __shared__ MlpLds L;
     if (rows_dev) rows = *rows_dev;  // row count held on the device
     const int64_t ntiles = (rows + 15) >> 4;
@@ -343,41 +365,70 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 #pragma unroll
             for (int t = 0; t < 4; t++) rh[t] = *reinterpret_cast<const f4*>(R + leaf * kE + 16 * t + 4 * g);
         }
-        // features 32 s + 8 g + j of this lane's row
+        // the lane's 32 features, x[8 s + j] = feature_of(s, g, j)
         float x[32];
-        const float* xr = X + (ok ? row : 0) * F + 8 * g;
+        const float* xr = X + (ok ? row : 0) * F;
+        auto load_row = [&]() {
 #pragma unroll
-        for (int p = 0; p < 16; p++) {
-            const int at = 32 * (p >> 2) + 2 * (p & 3);
-            float2 v = make_float2(0.0f, 0.0f);
-            if (ok && 8 * g + at < F) v = *reinterpret_cast<const float2*>(xr + at);
-            x[2 * p] = v.x;
-            x[2 * p + 1] = v.y;
-        }
-        // fc1
+            for (int p = 0; p < 16; p++) {
+                const int s = p >> 2, j = 2 * (p & 3);
+                const int at = s < 3 ? 16 * feature_section(s, j) + (j & 3) + 4 * g : 96 + j + 8 * g;
+                float2 v = make_float2(0.0f, 0.0f);
+                if (ok && at < F) v = *reinterpret_cast<const float2*>(xr + at);
+                x[2 * p] = v.x;
+                x[2 * p + 1] = v.y;
+            }
+        };
         f4 acc[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        // a feature past the parts' range (infinite, or rounding to it) has no
-        // split: its tile's first layer is summed plainly
-        float most = 0.0f;
+        const bool packed = !kRoot && units && rows > hw::kSuccStream;
+        if (packed) {
+            const uint32_t w = ok ? info[row] : 0u;
+            if (w & hw::kRowGeneral) {
+                load_row();
+            } else {
+                const hw::Unit& U = units[(ok ? row : 0) - (int64_t)(w & 255u)].u;
+                hw::Unit V;  // the fields a slice reads
+                V.cnt = U.cnt, V.hand = U.hand, V.near = U.near, V.pin = U.pin, V.dn = U.dn, V.bn = U.bn;
+                V.m = U.m, V.lift = U.lift, V.t = U.t;
+                float y[32];
+                hw::unit_slice(V, g, U.dsum[g], (w >> 8) & 15u, y);
 #pragma unroll
-        for (int j = 0; j < 32; j += 2) most = fmaxf(fmaxf(most, fabsf(x[j])), fabsf(x[j + 1]));
-        if (__ballot(most > kSplitMost)) {
-            for (int k = 0; k < F; k++) {
-                const float xk = ok ? X[row * F + k] : 0.0f;
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[t][i] += w1[(16 * t + 4 * g + i) * F + k] * xk;
+                for (int p = 0; p < 32; p++)
+                    x[p] = p < 24 ? y[4 * feature_section(p >> 3, p & 7) + (p & 3)] : y[p];
             }
-        } else {
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 b8 b[3];
                 split8([&](int j) { return x[8 * s + j]; }, b);
 #pragma unroll
-                for (int t = 0; t < 4; t++) acc[t] = mfma3(L.w1[s][t], lane, b, acc[t]);
+                for (int t = 0; t < 4; t++)
+                    acc[t] = s & 1 ? mfma3(L.w1[s][t], lane, b, acc[t]) : mfma3_whole(L.w1[s][t], lane, b[0], acc[t]);
+            }
+        } else {
+            load_row();
+            // a feature past the parts' range (infinite, or rounding to it) has no
+            // split: its tile's first layer is summed plainly
+            float most = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 32; j += 2) most = fmaxf(fmaxf(most, fabsf(x[j])), fabsf(x[j + 1]));
+            if (__ballot(most > kSplitMost)) {
+                for (int k = 0; k < F; k++) {
+                    const float xk = ok ? X[row * F + k] : 0.0f;
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[t][i] += w1[(16 * t + 4 * g + i) * F + k] * xk;
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    b8 b[3];
+                    split8([&](int j) { return x[8 * s + j]; }, b);
+#pragma unroll
+                    for (int t = 0; t < 4; t++) acc[t] = mfma3(L.w1[s][t], lane, b, acc[t]);
+                }
             }
         }
         // sigmoid + LayerNorm over the row's 64 units
@@ -560,6 +611,8 @@ int64_t hg_fnn_leaf_eval_lists_workspace(int64_t T, int F) {
     b += (T * kE + 2 * cap) * (int64_t)sizeof(float);     // root half of the action tower, logits, child values
     b = (b + 255) & ~(int64_t)255;
     b += (int64_t)sizeof(PackedNet);                      // the network in the kernels' LDS order
+    b = (b + 255) & ~(int64_t)255;
+    b += cap * (int64_t)(sizeof(hw::UnitRecord) + sizeof(uint32_t));  // unit records, a word per row
     return b;
 }
 
@@ -604,6 +657,9 @@ int leaf_eval_lists(const uint8_t* leaf_states, const uint8_t* legal_moves, cons
     off += (T * kE + 2 * cap) * (int64_t)sizeof(float);
     off = (off + 255) & ~(int64_t)255;
     PackedNet* pk = reinterpret_cast<PackedNet*>(base + off);
+    off = (off + (int64_t)sizeof(PackedNet) + 255) & ~(int64_t)255;
+    UnitRecord* units = reinterpret_cast<UnitRecord*>(base + off);
+    uint32_t* info = reinterpret_cast<uint32_t*>(units + cap);
     // plan, network layout and counters in one launch (the plan of a batch
     // over kPlanLeaves leaves takes its own two launches first)
     int plan_blocks = 0;
@@ -618,14 +674,14 @@ int leaf_eval_lists(const uint8_t* leaf_states, const uint8_t* legal_moves, cons
                        num_legal, T, plan_blocks, plan, fc1_w, F, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w,
                        action1_w, action1_b, action2_w, pk, leaf_idx, vl_lens,
                        reinterpret_cast<unsigned long long*>(stats));
-    int e = successor_rows_after_plan(leaf_states, legal_moves, T, workspace, X, st);
+    int e = successor_rows_after_plan(leaf_states, legal_moves, T, workspace, X, st, units, info);
     if (e) return e;
     hipLaunchKernelGGL(k_leaf_mlp<true>, dim3(mlp_blocks(T)), dim3(64 * kBlockWaves), 0, st, root_features, T, F,
                        nullptr, T, fc1_w, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, value_b, action1_w, action1_b,
                        action2_w, action2_b, R, root_values, nullptr, nullptr, pk);
     hipLaunchKernelGGL(k_leaf_mlp<false>, dim3(mlp_blocks(cap)), dim3(64 * kBlockWaves), 0, st, X, cap, F,
                        plan.a2r, T, fc1_w, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, value_b, action1_w, action1_b,
-                       action2_w, action2_b, R, cval, logit, plan.total, pk);
+                       action2_w, action2_b, R, cval, logit, plan.total, pk, units, info);
     hipLaunchKernelGGL(k_leaf_softmax, dim3(grid_for(T, 4)), dim3(256), 0, st, logit, cval, plan.offsets,
                        num_legal, T, priors, child_q, dense ? 1 : 0);
     return (int)hipGetLastError();

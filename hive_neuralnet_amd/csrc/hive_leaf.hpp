@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "hive_succ.hpp"
 #include "hive_wave.hpp"
 
 namespace hw {
@@ -80,11 +81,18 @@ inline RowsPlan rows_plan_of(void* workspace, int64_t T) {
     return RowsPlan{o, o + T, o + T + 1, o + T + 1 + T * kMaxLegal};
 }
 
+// Batches of at most kSuccStream rows go row by row, a lane group each
+// (successor_row): one row takes about a third of a pass's time.  Leaf
+// evaluation by rows / by passes, us: mid-game base game 14 K rows 65 / 73,
+// 27 K 88 / 76, 53 K 133 / 94; every piece 9 K rows 77 / 96, 19 K 104 / 102,
+// 38 K 155 / 110; after two plies 15 K 61 / 60, 31 K 73 / 61
+constexpr int kSuccStream = 18432;
+
 // hive_engine.hip: the plan of more than kPlanLeaves leaves (offsets, then the
 // row map), and the successor features of the planned rows
 int successor_rows_plan_large(const int32_t* num_legal, int64_t T, void* workspace, hipStream_t s);
 int successor_rows_after_plan(const uint8_t* states, const uint8_t* legal_moves, int64_t T, void* workspace,
-                              float* features, hipStream_t s);
+                              float* features, hipStream_t s, UnitRecord* units = nullptr, uint32_t* info = nullptr);
 
 // hive_fnn.hip: hg_fnn_leaf_eval_lists, and with `stats` (int64[4]) the
 // simulation wave's search counters of hg_mcts_wave_stats over leaf_idx,

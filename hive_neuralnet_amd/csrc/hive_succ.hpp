@@ -104,6 +104,7 @@ struct SuccBoard {
     uint16_t rtp[kWinRows];       // type and piece of each row of the window
     uint8_t runit[kWinRows];      // its unit
     uint16_t utp[kUnits], ufrom[kUnits], uto[kUnits];
+    uint8_t urow[kUnits];         // first row of each unit
     __device__ __forceinline__ Unit* units() { return reinterpret_cast<Unit*>(&P.u1); }
 };
 static_assert(offsetof(Pos, u2) == offsetof(Pos, u1) + sizeof(((Pos*)nullptr)->u1) &&
@@ -893,18 +894,18 @@ HW_INL void units_pass(SuccBoard& G, const SuccTables& K, const uint8_t* __restr
 // ---------------------------------------------------------------- rows
 // A quarter of a row's features: x[4 c + j] = feature 16 c + 4 g + j of the
 // six sections c of 16 classes, x[24 + j] = feature 96 + 8 g + j (past 121:
-// anything finite).  The four quarters run the same code -- lanes that differ
+// anything finite).  dsum: U.dsum[g].  The four quarters run the same code -- lanes that differ
 // in g do not diverge -- and are what the lane groups of the network's first
 // product take.  k: the class that a placement's row adds.  Divisions rounded
 // as features_finish rounds them (div_exact).
-HW_INL void unit_slice(const Unit& U, int g, uint32_t k, float* x) {
+HW_INL void unit_slice(const Unit& U, int g, uint32_t dsum, uint32_t k, float* x) {
     const uint32_t m = U.m;
     const bool add = (m & kUPlace) != 0;
     const uint32_t one = add ? 1u << (2 * k) : 0u;
     const uint32_t cnt = (U.cnt + one) >> (8 * g), hand = (U.hand - one) >> (8 * g);
     const uint32_t near = (U.near + ((m & kUNear) ? one : 0u)) >> (8 * g);
     const uint32_t dn = (U.dn + ((m & kUDist) ? one : 0u)) >> (8 * g);
-    const uint32_t ds = U.dsum[g] + ((m & kUDist) && (k >> 2) == (uint32_t)g ? (U.t >> 16) << (8 * (k & 3)) : 0u);
+    const uint32_t ds = dsum + ((m & kUDist) && (k >> 2) == (uint32_t)g ? (U.t >> 16) << (8 * (k & 3)) : 0u);
     const uint32_t move = U.bn >> (4 * g), pin = U.pin >> (8 * g);
     // hands by the pieces of a set: types 2 g and 2 g + 1 of 1 3 3 2 2 1 1 1
     const float pa = g == 1 ? 3.0f : g == 2 ? 2.0f : 1.0f, ra = g == 1 ? 1.f / 3.f : g == 2 ? 0.5f : 1.0f;
@@ -942,6 +943,29 @@ HW_INL void unit_slice(const Unit& U, int g, uint32_t k, float* x) {
 // no feature is one) until general_range has written it.
 constexpr uint32_t kGeneralMark = 0xFFFFFFFFu;
 
+// What a window's rows leave behind.  FeatureRows: 122 floats a row, eight
+// rows at a time, four lanes each.  UnitRows: the units' records at their first
+// rows, and a word per row -- rows back to the record, the class a placement's
+// row adds at bit 8, kRowGeneral -- from which the network builds its operands
+// (unit_slice); feat then holds the rows of the general program only.
+struct FeatureRows {
+    float* feat;
+};
+struct alignas(64) UnitRecord {
+    Unit u;
+    uint32_t pad[3];
+};
+constexpr uint32_t kRowGeneral = 1u << 31;
+struct UnitRows {
+    float* feat;
+    UnitRecord* units;
+    uint32_t* info;
+};
+template <class Out>
+constexpr bool kToUnits = false;
+template <>
+inline constexpr bool kToUnits<UnitRows> = true;
+
 // Where a row's root and slot come from: maps over the batch, or a list's rows
 // in slot order (one memory round trip less).
 struct MapRows {
@@ -966,10 +990,10 @@ struct ListRows {
 // number of windows.  A row whose root or slot is out of range gets zero
 // features; a child outside what the units cover (a board or move no game
 // reaches) is marked, and the return value says that the range has such rows.
-template <typename Ix, class Rows>
+template <typename Ix, class Rows, class Out>
 HW_INL bool successor_range(SuccBoard& G, const SuccTables& K, const uint8_t* __restrict__ states,
                             const uint8_t* __restrict__ legal, const Rows& src, Ix lo, Ix hi, int64_t num_roots,
-                            const uint8_t* __restrict__ zero_row, int wave_lane, float* feat_out) {
+                            const uint8_t* __restrict__ zero_row, int wave_lane, const Out& dst) {
     int64_t cur = -2;  // the root whose tables are in LDS
     bool general = false;
     Ix at = lo;
@@ -1038,39 +1062,59 @@ HW_INL bool successor_range(SuccBoard& G, const SuccTables& K, const uint8_t* __
                 G.utp[u] = (uint16_t)tp[j];
                 G.ufrom[u] = (uint16_t)from[j];
                 G.uto[u] = (uint16_t)to[j];
+                G.urow[u] = (uint8_t)(kW * j + l);
             }
         }
         __syncthreads();
         units_pass(G, K, S, lane, nu);
 
-        // -- rows: eight at a time, four lanes each
-        const int g = l & 3;
         const uint32_t me = G.P.turn & 1;
-        for (int r0 = 0; hw_wave_any(r0 < rows); r0 += 8) {
-            const int r = r0 + (l >> 2);
-            if (r >= rows) continue;
-            float* out = feat_out + (Ix)((at + (Ix)r) * (Ix)kFeat);
-            float x[32];
-            if (work) {
-                const Unit& U = G.units()[G.runit[r]];
-                if (U.m & kUGeneral) {
+        if constexpr (kToUnits<Out>) {
+            if (l < nu) {
+                const Unit& U = G.units()[l];
+                if (!(U.m & kUGeneral)) dst.units[at + (Ix)G.urow[l]].u = U;
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int r = kW * j + l;
+                if (r >= rows) continue;
+                const int u = work ? G.runit[r] : 0;
+                const bool gen = !work || (G.units()[u].m & kUGeneral);
+                const uint32_t k = (((uint32_t)(G.rtp[r] >> 8) - 1u) * 2u + me) & 15u;
+                dst.info[at + (Ix)r] = gen ? kRowGeneral : (uint32_t)(r - G.urow[u]) | (k << 8);
+                if (gen) {
                     general = true;
-                    if (g == 0) *reinterpret_cast<uint32_t*>(out) = kGeneralMark;
-                    continue;
+                    reinterpret_cast<uint32_t*>(dst.feat)[(Ix)((at + (Ix)r) * (Ix)kFeat)] = kGeneralMark;
                 }
-                unit_slice(U, g, (((uint32_t)(G.rtp[r] >> 8) - 1u) * 2u + me) & 15u, x);
-            } else {  // rows of no root or slot
-#pragma unroll
-                for (int k = 0; k < 32; k++) x[k] = 0.0f;
             }
+        } else {
+            const int g = l & 3;
+            for (int r0 = 0; hw_wave_any(r0 < rows); r0 += 8) {
+                const int r = r0 + (l >> 2);
+                if (r >= rows) continue;
+                float* out = dst.feat + (Ix)((at + (Ix)r) * (Ix)kFeat);
+                float x[32];
+                if (work) {
+                    const Unit& U = G.units()[G.runit[r]];
+                    if (U.m & kUGeneral) {
+                        general = true;
+                        if (g == 0) *reinterpret_cast<uint32_t*>(out) = kGeneralMark;
+                        continue;
+                    }
+                    unit_slice(U, g, U.dsum[g], (((uint32_t)(G.rtp[r] >> 8) - 1u) * 2u + me) & 15u, x);
+                } else {  // rows of no root or slot
 #pragma unroll
-            for (int c = 0; c < 6; c++) {
-                *reinterpret_cast<f32x2*>(out + 16 * c + 4 * g) = f32x2{x[4 * c], x[4 * c + 1]};
-                *reinterpret_cast<f32x2*>(out + 16 * c + 4 * g + 2) = f32x2{x[4 * c + 2], x[4 * c + 3]};
+                    for (int k = 0; k < 32; k++) x[k] = 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < 6; c++) {
+                    *reinterpret_cast<f32x2*>(out + 16 * c + 4 * g) = f32x2{x[4 * c], x[4 * c + 1]};
+                    *reinterpret_cast<f32x2*>(out + 16 * c + 4 * g + 2) = f32x2{x[4 * c + 2], x[4 * c + 3]};
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j += 2)
+                    if (j < 2 || g < 3) *reinterpret_cast<f32x2*>(out + 96 + 8 * g + j) = f32x2{x[24 + j], x[25 + j]};
             }
-#pragma unroll
-            for (int j = 0; j < 8; j += 2)
-                if (j < 2 || g < 3) *reinterpret_cast<f32x2*>(out + 96 + 8 * g + j) = f32x2{x[24 + j], x[25 + j]};
         }
         __syncthreads();
         at += (Ix)rows;

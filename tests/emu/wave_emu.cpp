@@ -94,11 +94,45 @@ void emu_successor_units(const uint8_t* states, const uint8_t* legal, const int6
         const int64_t q = r * kPosPerWave + t / kW;
         const int64_t lo = std::min(N, q * per), hi = std::min(N, lo + per);
         const bool general = successor_range<int64_t>(g_succ[t / kW], kSuccTables, states, legal,
-                                                      MapRows{a2r, midx}, lo, hi, num_roots, zero_row, t, feat);
+                                                      MapRows{a2r, midx}, lo, hi, num_roots, zero_row, t,
+                                                      FeatureRows{feat});
         __syncthreads();
         if (hw_wave_any(general))
             general_range<int64_t>(g_succ[t / kW], states, legal, a2r, midx, lo, hi, num_roots, zero_row, t, feat);
     });
+}
+// The same with the rows left as units, each row's features then built from its
+// record in four quarters as the network's lanes build them (midx: the slots in
+// list order, as the leaf evaluation's plan lists them).
+void emu_successor_records(const uint8_t* states, const uint8_t* legal, const int64_t* a2r, const int64_t* midx,
+                           int64_t N, int64_t num_roots, int64_t per, float* feat) {
+    static const uint8_t zero_row[kStateBytes] = {};
+    memset(g_succ, 0xA5, sizeof g_succ);
+    std::vector<UnitRecord> units(N);
+    std::vector<uint32_t> info(N, 0);
+    const UnitRows out{feat, units.data(), info.data()};
+    const int64_t ranges = (N + per - 1) / per;
+    run_group(64, (ranges + kPosPerWave - 1) / kPosPerWave, [&](int64_t r, int t) {
+        const int64_t q = r * kPosPerWave + t / kW;
+        const int64_t lo = std::min(N, q * per), hi = std::min(N, lo + per);
+        const bool general = successor_range<int64_t>(g_succ[t / kW], kSuccTables, states, legal,
+                                                      MapRows{a2r, midx}, lo, hi, num_roots, zero_row, t, out);
+        __syncthreads();
+        if (hw_wave_any(general))
+            general_range<int64_t>(g_succ[t / kW], states, legal, a2r, midx, lo, hi, num_roots, zero_row, t, feat);
+    });
+    for (int64_t i = 0; i < N; i++) {
+        if (info[i] & kRowGeneral) continue;
+        const Unit& U = units[i - (info[i] & 255u)].u;
+        for (int g = 0; g < 4; g++) {
+            float x[32];
+            unit_slice(U, g, U.dsum[g], (info[i] >> 8) & 15u, x);
+            for (int e = 0; e < 32; e++) {
+                const int f = e < 24 ? 16 * (e >> 2) + 4 * g + (e & 3) : 96 + 8 * g + (e - 24);
+                if (f < kFeat) feat[i * kFeat + f] = x[e];
+            }
+        }
+    }
 }
 // k_random_play's ply loop with given choices: game i's board is loaded
 // once, then per ply (while its result is 0) the derived tables are rebuilt,

@@ -234,9 +234,9 @@ def _all_rows(n):
     return roots, np.concatenate([np.arange(int(k), dtype=np.int64) for k in n])
 
 
-def _units(emu, st, mv, roots, idx, per):
+def _units(emu, st, mv, roots, idx, per, records=False):
     f = np.full((len(roots), 122), np.nan, np.float32)
-    emu.emu_successor_units(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
+    (emu.emu_successor_records if records else emu.emu_successor_units)(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
                             ctypes.c_int64(st.shape[0]), ctypes.c_int64(per), _p(f))
     return f
 
@@ -253,8 +253,9 @@ def test_emulated_successor_units(emu, oracle, mask, max_ply, per):
     mv = np.ascontiguousarray(mv)
     roots, idx = _all_rows(n)
     want = oracle.batch_successor_features(st, mv, roots, idx)
-    got = _units(emu, st, mv, roots, idx, per)
-    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    for records in (False, True):  # rows as features, and as the units the network reads
+        got = _units(emu, st, mv, roots, idx, per, records)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), records
 
 
 def test_emulated_successor_units_any_rows(emu, oracle):
@@ -285,6 +286,7 @@ def test_emulated_successor_units_any_rows(emu, oracle):
     emu.emu_successor_rows(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
                            ctypes.c_int64(st.shape[0]), _p(want))
     got = _units(emu, st, mv, roots, idx, 50)
+    assert np.array_equal(_units(emu, st, mv, roots, idx, 50, True).view(np.uint32), got.view(np.uint32))
     bad = np.nonzero((got.view(np.uint32) != want.view(np.uint32)).any(1))[0]
     assert len(bad) == 0, [(int(r), mv[roots[r] % len(st), idx[r] % 256].tolist(),
                             np.nonzero(got[r] != want[r])[0].tolist()) for r in bad[:6]]

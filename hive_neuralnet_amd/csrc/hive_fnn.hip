@@ -174,17 +174,16 @@ constexpr int kPackBlocks = (kPackThreads + 255) / 256;
 // and, with `stats`, the simulation wave's search counters (one block per
 // 1,024 simulations: leaves reached, their legal counts, their virtual-loss
 // lengths, rows; integer sums added with device atomics).
-__global__ __launch_bounds__(256) void k_leaf_prep(const int32_t* __restrict__ nlegal, int64_t T, int plan_blocks,
-                                                   hw::RowsPlan plan, const float* __restrict__ w1, int F,
-                                                   const float* __restrict__ b1, const float* __restrict__ lnw,
-                                                   const float* __restrict__ lnb, const float* __restrict__ w2,
-                                                   const float* __restrict__ b2, const float* __restrict__ wv,
-                                                   const float* __restrict__ a1w, const float* __restrict__ a1b,
-                                                   const float* __restrict__ a2w, PackedNet* __restrict__ pk,
-                                                   const int32_t* __restrict__ leaf_idx,
-                                                   const int32_t* __restrict__ vl_lens,
-                                                   unsigned long long* __restrict__ stats) {
-    int b = (int)blockIdx.x;
+__device__ __forceinline__ void leaf_prep(int b, const int32_t* __restrict__ nlegal, int64_t T, int plan_blocks,
+    hw::RowsPlan plan, const float* __restrict__ w1, int F,
+    const float* __restrict__ b1, const float* __restrict__ lnw,
+    const float* __restrict__ lnb, const float* __restrict__ w2,
+    const float* __restrict__ b2, const float* __restrict__ wv,
+    const float* __restrict__ a1w, const float* __restrict__ a1b,
+    const float* __restrict__ a2w, PackedNet* __restrict__ pk,
+    const int32_t* __restrict__ leaf_idx,
+    const int32_t* __restrict__ vl_lens,
+    unsigned long long* __restrict__ stats) {
     if (b < plan_blocks) {
         hw::rows_plan_block(nlegal, T, plan.offsets, plan.total, plan.a2r, plan.mi, b);
         return;
@@ -223,6 +222,19 @@ __global__ __launch_bounds__(256) void k_leaf_prep(const int32_t* __restrict__ n
     } else if (tid == 3 && b == 0) {
         atomicAdd(&stats[3], (unsigned long long)T);
     }
+}
+
+__global__ __launch_bounds__(256) void k_leaf_prep(const int32_t* __restrict__ nlegal, int64_t T, int plan_blocks,
+    hw::RowsPlan plan, const float* __restrict__ w1, int F,
+    const float* __restrict__ b1, const float* __restrict__ lnw,
+    const float* __restrict__ lnb, const float* __restrict__ w2,
+    const float* __restrict__ b2, const float* __restrict__ wv,
+    const float* __restrict__ a1w, const float* __restrict__ a1b,
+    const float* __restrict__ a2w, PackedNet* __restrict__ pk,
+    const int32_t* __restrict__ leaf_idx,
+    const int32_t* __restrict__ vl_lens,
+    unsigned long long* __restrict__ stats) {
+    leaf_prep((int)blockIdx.x, nlegal, T, plan_blocks, plan, w1, F, b1, lnw, lnb, w2, b2, wv, a1w, a1b, a2w, pk, leaf_idx, vl_lens, stats);
 }
 
 // sigmoid from the hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32):
@@ -282,25 +294,24 @@ __device__ __forceinline__ f4 vec4(const MlpLds& L, int which, int t, int g) {
 //         and more than kSuccStream rows the features come from the rows' unit
 //         records (X holds the rows marked kRowGeneral only).
 template <bool kRoot>
-__global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __restrict__ X, int64_t rows, int F,
-                                                  const int64_t* __restrict__ succ_leaf, int64_t T,
-                                                  const float* __restrict__ w1, const float* __restrict__ b1,
-                                                  const float* __restrict__ lnw, const float* __restrict__ lnb,
-                                                  const float* __restrict__ w2, const float* __restrict__ b2,
-                                                  const float* __restrict__ wv, float bv, const float* __restrict__ a1w,
-                                                  const float* __restrict__ a1b, const float* __restrict__ a2w, float ba2,
-                                                  float* __restrict__ R, float* __restrict__ value,
-                                                  float* __restrict__ logit, const int64_t* __restrict__ rows_dev,
-                                                  const PackedNet* __restrict__ pk,
-                                                  const hw::UnitRecord* __restrict__ units = nullptr,
-                                                  const uint32_t* __restrict__ info = nullptr) {
-    __shared__ MlpLds L;
+__device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t blocks, const float* __restrict__ X, int64_t rows, int F,
+                                         const int64_t* __restrict__ succ_leaf, int64_t T,
+                                         const float* __restrict__ w1, const float* __restrict__ b1,
+                                         const float* __restrict__ lnw, const float* __restrict__ lnb,
+                                         const float* __restrict__ w2, const float* __restrict__ b2,
+                                         const float* __restrict__ wv, float bv, const float* __restrict__ a1w,
+                                         const float* __restrict__ a1b, const float* __restrict__ a2w, float ba2,
+                                         float* __restrict__ R, float* __restrict__ value,
+                                         float* __restrict__ logit, const int64_t* __restrict__ rows_dev,
+                                         const PackedNet* __restrict__ pk,
+                                         const hw::UnitRecord* __restrict__ units,
+                                         const uint32_t* __restrict__ info) {
     if (rows_dev) rows = *rows_dev;  // row count held on the device
     const int64_t ntiles = (rows + 15) >> 4;
     // 16-row tiles dealt over the blocks first (tile = block + grid * (wave +
     // kBlockWaves * round)): a short batch spreads over all CUs, and a block
     // with no tile leaves before filling LDS
-    if ((int64_t)blockIdx.x >= ntiles) return;
+    if (block >= ntiles) return;
     if (pk) {  // the packed layout: straight 16-byte copies, every load issued before the first store
         constexpr int kT = 64 * kBlockWaves, k12 = (sizeof(L.w1) + sizeof(L.w2)) / 16, k3 = sizeof(L.w3) / 16;
         constexpr int n12 = (k12 + kT - 1) / kT, n3 = (k3 + kT - 1) / kT;
@@ -325,16 +336,32 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
         for (int k = 0; k < n3; k++)
             if (tid + k * kT < k3) d3[tid + k * kT] = c3[k];
         if (tid < 7 * kE / 4) reinterpret_cast<f4*>(&L.vec[0][0])[tid] = cv;
-    } else {  // weights gathered, permuted and split into LDS (perm_index)
+    } else {  // weights gathered, permuted and split into LDS (perm_index), every load issued before the first split
+        constexpr int kT = 64 * kBlockWaves, n1 = kPack1 / kT, n2 = kPack2 / kT;
+        static_assert(kPack1 % kT == 0 && kPack2 % kT == 0, "whole rounds");
+        float c1[n1], c2[n2], c3[n2];
         int m, k, at;
-        for (int i = threadIdx.x; i < kPack1; i += blockDim.x) {
-            perm_index(i, true, m, k, at);
-            put_split(reinterpret_cast<__bf16*>(&L.w1), at, k < F ? w1[m * F + k] : 0.0f);
+#pragma unroll
+        for (int q = 0; q < n1; q++) {
+            perm_index(threadIdx.x + q * kT, true, m, k, at);
+            c1[q] = k < F ? w1[m * F + k] : 0.0f;
         }
-        for (int i = threadIdx.x; i < kPack2; i += blockDim.x) {
-            perm_index(i, false, m, k, at);
-            put_split(reinterpret_cast<__bf16*>(&L.w2), at, w2[m * kE + k]);
-            put_split(reinterpret_cast<__bf16*>(&L.w3), at, a1w[m * 2 * kE + (kRoot ? 0 : kE) + k]);
+#pragma unroll
+        for (int q = 0; q < n2; q++) {
+            perm_index(threadIdx.x + q * kT, false, m, k, at);
+            c2[q] = w2[m * kE + k];
+            c3[q] = a1w[m * 2 * kE + (kRoot ? 0 : kE) + k];
+        }
+#pragma unroll
+        for (int q = 0; q < n1; q++) {
+            perm_index(threadIdx.x + q * kT, true, m, k, at);
+            put_split(reinterpret_cast<__bf16*>(&L.w1), at, c1[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < n2; q++) {
+            perm_index(threadIdx.x + q * kT, false, m, k, at);
+            put_split(reinterpret_cast<__bf16*>(&L.w2), at, c2[q]);
+            put_split(reinterpret_cast<__bf16*>(&L.w3), at, c3[q]);
         }
         if (threadIdx.x < kE) {
             const int u = threadIdx.x;
@@ -350,8 +377,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
     __syncthreads();
 
     const int lane = threadIdx.x & 63, g = lane >> 4;
-    for (int64_t tile = (int64_t)blockIdx.x + (int64_t)gridDim.x * (threadIdx.x >> 6); tile < ntiles;
-         tile += (int64_t)gridDim.x * kBlockWaves) {
+    for (int64_t tile = block + blocks * (threadIdx.x >> 6); tile < ntiles; tile += blocks * kBlockWaves) {
         // the weights are re-read from LDS in every tile: hoisted out of the
         // loop they would take hundreds of registers and leave one wave per SIMD
         __asm__ volatile("" ::: "memory");
@@ -515,6 +541,48 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
     }
 }
 
+template <bool kRoot>
+__global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __restrict__ X, int64_t rows, int F,
+                                                  const int64_t* __restrict__ succ_leaf, int64_t T,
+                                                  const float* __restrict__ w1, const float* __restrict__ b1,
+                                                  const float* __restrict__ lnw, const float* __restrict__ lnb,
+                                                  const float* __restrict__ w2, const float* __restrict__ b2,
+                                                  const float* __restrict__ wv, float bv, const float* __restrict__ a1w,
+                                                  const float* __restrict__ a1b, const float* __restrict__ a2w, float ba2,
+                                                  float* __restrict__ R, float* __restrict__ value,
+                                                  float* __restrict__ logit, const int64_t* __restrict__ rows_dev,
+                                                  const PackedNet* __restrict__ pk,
+                                                  const hw::UnitRecord* __restrict__ units = nullptr,
+                                                  const uint32_t* __restrict__ info = nullptr) {
+    __shared__ MlpLds L;
+    leaf_mlp<kRoot>(L, blockIdx.x, gridDim.x, X, rows, F, succ_leaf, T, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R, value, logit, rows_dev, pk, units, info);
+}
+
+// The first launch of a short evaluation: k_leaf_prep's blocks (their first 256
+// threads) beside the root rows' tiles, whose blocks take the weights from the
+// network itself instead of waiting for the packed ones.  Every block fits the
+// chip at once (one per CU) up to kFirstLeaves leaves: 128 tile blocks, 81 of
+// packing, the plan's and the counters'.
+constexpr int64_t kFirstLeaves = 2048;
+__global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_first(
+    int root_blocks, const float* __restrict__ X, int64_t T, int F, hw::RowsPlan plan, int plan_blocks,
+    const int32_t* __restrict__ nlegal, const float* __restrict__ w1, const float* __restrict__ b1,
+    const float* __restrict__ lnw, const float* __restrict__ lnb, const float* __restrict__ w2,
+    const float* __restrict__ b2, const float* __restrict__ wv, float bv, const float* __restrict__ a1w,
+    const float* __restrict__ a1b, const float* __restrict__ a2w, float ba2, PackedNet* __restrict__ pk,
+    float* __restrict__ R, float* __restrict__ value, const int32_t* __restrict__ leaf_idx,
+    const int32_t* __restrict__ vl_lens, unsigned long long* __restrict__ stats) {
+    __shared__ MlpLds L;
+    if ((int)blockIdx.x < root_blocks) {
+        leaf_mlp<true>(L, blockIdx.x, root_blocks, X, T, F, nullptr, T, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w,
+                       ba2, R, value, nullptr, nullptr, nullptr, nullptr, nullptr);
+        return;
+    }
+    if (threadIdx.x >= 256) return;  // whole waves: the barriers below count the others
+    leaf_prep((int)blockIdx.x - root_blocks, nlegal, T, plan_blocks, plan, w1, F, b1, lnw, lnb, w2, b2, wv, a1w, a1b,
+              a2w, pk, leaf_idx, vl_lens, stats);
+}
+
 __device__ __forceinline__ float wave_sum_f(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -670,15 +738,26 @@ int leaf_eval_lists(const uint8_t* leaf_states, const uint8_t* legal_moves, cons
         if (e) return e;
     }
     const int stat_blocks = stats ? (int)((T + 1023) / 1024) : 0;
-    hipLaunchKernelGGL(k_leaf_prep, dim3((unsigned)(plan_blocks + kPackBlocks + stat_blocks)), dim3(256), 0, st,
-                       num_legal, T, plan_blocks, plan, fc1_w, F, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w,
-                       action1_w, action1_b, action2_w, pk, leaf_idx, vl_lens,
-                       reinterpret_cast<unsigned long long*>(stats));
+    const int prep_blocks = plan_blocks + kPackBlocks + stat_blocks;
+    unsigned long long* counters = reinterpret_cast<unsigned long long*>(stats);
+    const bool first = T <= kFirstLeaves;
+    if (first) {
+        const int root_blocks = mlp_blocks(T);
+        hipLaunchKernelGGL(k_leaf_first, dim3((unsigned)(root_blocks + prep_blocks)), dim3(64 * kBlockWaves), 0, st,
+                           root_blocks, root_features, T, F, plan, plan_blocks, num_legal, fc1_w, fc1_b, ln_w, ln_b,
+                           fc2_w, fc2_b, value_w, value_b, action1_w, action1_b, action2_w, action2_b, pk, R,
+                           root_values, leaf_idx, vl_lens, counters);
+    } else {
+        hipLaunchKernelGGL(k_leaf_prep, dim3((unsigned)prep_blocks), dim3(256), 0, st, num_legal, T, plan_blocks, plan,
+                           fc1_w, F, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, action1_w, action1_b, action2_w, pk,
+                           leaf_idx, vl_lens, counters);
+    }
     int e = successor_rows_after_plan(leaf_states, legal_moves, T, workspace, X, st, units, info);
     if (e) return e;
-    hipLaunchKernelGGL(k_leaf_mlp<true>, dim3(mlp_blocks(T)), dim3(64 * kBlockWaves), 0, st, root_features, T, F,
-                       nullptr, T, fc1_w, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, value_b, action1_w, action1_b,
-                       action2_w, action2_b, R, root_values, nullptr, nullptr, pk);
+    if (!first)
+        hipLaunchKernelGGL(k_leaf_mlp<true>, dim3(mlp_blocks(T)), dim3(64 * kBlockWaves), 0, st, root_features, T, F,
+                           nullptr, T, fc1_w, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, value_b, action1_w, action1_b,
+                           action2_w, action2_b, R, root_values, nullptr, nullptr, pk);
     hipLaunchKernelGGL(k_leaf_mlp<false>, dim3(mlp_blocks(cap)), dim3(64 * kBlockWaves), 0, st, X, cap, F,
                        plan.a2r, T, fc1_w, fc1_b, ln_w, ln_b, fc2_w, fc2_b, value_w, value_b, action1_w, action1_b,
                        action2_w, action2_b, R, cval, logit, plan.total, pk, units, info);

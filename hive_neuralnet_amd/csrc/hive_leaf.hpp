@@ -83,10 +83,10 @@ inline RowsPlan rows_plan_of(void* workspace, int64_t T) {
 
 // Batches of at most kSuccStream rows go row by row, a lane group each
 // (successor_row): one row takes about a third of a pass's time.  Leaf
-// evaluation by rows / by passes, us: mid-game base game 14 K rows 65 / 73,
-// 27 K 88 / 76, 53 K 133 / 94; every piece 9 K rows 77 / 96, 19 K 104 / 102,
-// 38 K 155 / 110; after two plies 15 K 61 / 60, 31 K 73 / 61
-constexpr int kSuccStream = 18432;
+// evaluation by rows / by passes, us: mid-game base game 14 K rows 61 / 65,
+// 21 K 74 / 67, 53 K 124 / 77; every piece 14 K 81 / 92, 19 K 101 / 95, 38 K
+// 150 / 97
+constexpr int kSuccStream = 16384;
 
 // hive_engine.hip: the plan of more than kPlanLeaves leaves (offsets, then the
 // row map), and the successor features of the planned rows

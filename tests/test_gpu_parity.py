@@ -372,10 +372,10 @@ def test_random_play_pair_counter_scratch(ext):
         assert torch.equal(st, want_states) and torch.equal(plies, want_plies)
 
 
-@pytest.mark.parametrize("mask,rows", [(0, 18432), (0, 18433), (7, 18465)])
+@pytest.mark.parametrize("mask,rows", [(0, 16384), (0, 16385), (7, 16417)])
 def test_successor_rows_both_programs(ext, oracle, mask, rows):
     """Successor features on both sides of the row count from which a batch's
-    children are worked out one lane each (18,432), rows of whole lists then
+    children are worked out one lane each (16,384), rows of whole lists then
     rows in random order with some out of range, against the oracle."""
     st, _ = oracle.generate_positions(420, mask, 120, 4100 + mask)
     mv, n, _, _ = oracle.batch_legal_features_actions(st)

@@ -201,9 +201,10 @@ def _select_outputs(T: int, whole_rows: bool = False):
 
 # fused lists of more positions than this are taken in turn order: up to here the
 # device holds nearly every position at once, and the order costs a launch
-# (ordered / index order, us: 1 position 25 / 22, 4,096 37 / 32, 8,192 42 / 39,
-# 12,288 55 / 59; with every piece 8,192 104 / 98, 12,288 113 / 125)
-_order_min_batch = 10240
+# (ordered / index order, us: 1 position 25 / 22, 4,000 base 34-37 / 31-33, every
+# piece 93-98 / 86-93; 7,001 of at most 30 plies 35.2 / 35.6; 10,240 of at most 30
+# plies 37 / 40, of at most 145 45 / 43)
+_order_min_batch = 6144
 
 _lib = None
 _lib_lock = threading.Lock()

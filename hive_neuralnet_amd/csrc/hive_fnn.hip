@@ -29,10 +29,13 @@
 // instruction; what is left out is a quarter of a float32 rounding.  The
 // weights are split once per evaluation, the activations as they come.
 // Measured against the fp32 instruction (427 K successor rows): 143 -> 91 us,
-// and the outputs' distance from float64 the same (1.4e-7 / 1.4e-7 to 8.5e-7 /
-// 7.7e-7 relative over the seeds tried).  Bound now by the element-wise work
-// (~800 VALU a tile), the matrix pipe and 96 KB of LDS reads a tile, about
-// equal parts.
+// 78 us with the units' records for features, the sums started from the biases
+// and fused multiply-adds around the products; the outputs' distance from
+// float64 is the same (1.4e-7 / 1.4e-7 to 8.5e-7 / 7.7e-7 relative over the seeds
+// tried).  Bound now by VALU issue (~750 a tile, a third of it the splits) and
+// the matrix pipe (168 instructions a tile), which add up to about the time
+// measured; not by the 96 KB of LDS reads a tile: two tiles per read took as
+// long (85.7 us against 85.9 before the multiply-adds).
 //
 // Matrix-core layout (16x16x32, D = A.B + C, A 16x32, B 32x16): lane l holds
 // A[l%16][8 (l/16) + j], B[8 (l/16) + j][l%16] (j < 8) and D[4(l/16)+i][l%16]
@@ -383,13 +386,14 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
         __asm__ volatile("" ::: "memory");
         const int64_t row = tile * 16 + (lane & 15);
         const bool ok = row < rows;
-        // successor rows: the leaf's root half of the action tower, fetched first
+        // successor rows: the leaf's root half of the action tower, fetched once the
+        // features' registers are free (before them 14 registers spill)
         f4 rh[4];
+        const float* half = nullptr;
         if constexpr (!kRoot) {
             int64_t leaf = ok ? succ_leaf[row] : 0;
             leaf = leaf < 0 ? 0 : (leaf >= T ? T - 1 : leaf);
-#pragma unroll
-            for (int t = 0; t < 4; t++) rh[t] = *reinterpret_cast<const f4*>(R + leaf * kE + 16 * t + 4 * g);
+            half = R + leaf * kE + 4 * g;
         }
         // the lane's 32 features, x[8 s + j] = feature_of(s, g, j)
         float x[32];
@@ -405,9 +409,9 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
                 x[2 * p + 1] = v.y;
             }
         };
-        f4 acc[4];
+        f4 acc[4];  // every layer's sums start from its bias
 #pragma unroll
-        for (int t = 0; t < 4; t++) acc[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < 4; t++) acc[t] = vec4(L, kB1, t, g);
         const bool packed = !kRoot && units && rows > hw::kSuccStream;
         if (packed) {
             const uint32_t w = ok ? info[row] : 0u;
@@ -457,17 +461,19 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
                 }
             }
         }
+        if constexpr (!kRoot) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) rh[t] = *reinterpret_cast<const f4*>(half + 16 * t);
+        }
         // sigmoid + LayerNorm over the row's 64 units
         float sum = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const f4 b = vec4(L, kB1, t, g);
+        for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                acc[t][i] = sigmoidf_(acc[t][i] + b[i]);
+                acc[t][i] = sigmoidf_(acc[t][i]);
                 sum += acc[t][i];
             }
-        }
         const float mean = row_sum(sum) / (float)kE;
         float sq = 0.0f;
 #pragma unroll
@@ -475,19 +481,19 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 acc[t][i] -= mean;
-                sq += acc[t][i] * acc[t][i];
+                sq = __builtin_fmaf(acc[t][i], acc[t][i], sq);
             }
-        const float rstd = 1.0f / sqrtf(row_sum(sq) / (float)kE + 1e-5f);
+        const float rstd = __builtin_amdgcn_rsqf(row_sum(sq) / (float)kE + 1e-5f);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const f4 w = vec4(L, kLnW, t, g), b = vec4(L, kLnB, t, g);
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[t][i] = acc[t][i] * rstd * w[i] + b[i];
+            for (int i = 0; i < 4; i++) acc[t][i] = __builtin_fmaf(acc[t][i] * rstd, w[i], b[i]);
         }
         // fc2 -> embedding
         f4 e[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) e[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < 4; t++) e[t] = vec4(L, kB2, t, g);
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             b8 b[3];
@@ -498,18 +504,18 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
         float v = 0.0f;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            const f4 b = vec4(L, kB2, t, g), w = vec4(L, kWv, t, g);
+            const f4 w = vec4(L, kWv, t, g);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                e[t][i] += b[i];
-                v += e[t][i] * w[i];
-            }
+            for (int i = 0; i < 4; i++) v = __builtin_fmaf(e[t][i], w[i], v);
         }
         v = tanhf(row_sum(v) + bv);
         // action tower, first layer (root or successor half)
         f4 h[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) h[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < 4; t++) {
+            if constexpr (kRoot) h[t] = vec4(L, kBa1, t, g);
+            else h[t] = rh[t];
+        }
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             b8 b[3];
@@ -521,7 +527,7 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
             if (ok) {
 #pragma unroll
                 for (int t = 0; t < 4; t++)
-                    *reinterpret_cast<f4*>(R + row * kE + 16 * t + 4 * g) = h[t] + vec4(L, kBa1, t, g);
+                    *reinterpret_cast<f4*>(R + row * kE + 16 * t + 4 * g) = h[t];
                 if (g == 0) value[row] = v;
             }
         } else {
@@ -530,7 +536,7 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
             for (int t = 0; t < 4; t++) {
                 const f4 w = vec4(L, kWa2, t, g);
 #pragma unroll
-                for (int i = 0; i < 4; i++) a += sigmoidf_(h[t][i] + rh[t][i]) * w[i];
+                for (int i = 0; i < 4; i++) a = __builtin_fmaf(sigmoidf_(h[t][i]), w[i], a);
             }
             a = row_sum(a) + ba2;
             if (ok && g == 0) {

@@ -568,7 +568,8 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 // threads) beside the root rows' tiles, whose blocks take the weights from the
 // network itself instead of waiting for the packed ones.  Every block fits the
 // chip at once (one per CU) up to kFirstLeaves leaves: 128 tile blocks, 81 of
-// packing, the plan's and the counters'.
+// packing, the plan's and the counters'.  Base-game leaf evaluation: 2,048 leaves
+// 83 us, 2,100 (the leaf rows' network in a launch of its own) 100 us.
 constexpr int64_t kFirstLeaves = 2048;
 __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_first(
     int root_blocks, const float* __restrict__ X, int64_t T, int F, hw::RowsPlan plan, int plan_blocks,

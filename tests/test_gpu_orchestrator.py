@@ -764,3 +764,25 @@ def test_leaf_eval_products_against_float64(T, each, scale):
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     ok = torch.isfinite(want)
     assert float((got[ok] - want[ok]).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("T,ply", [(1, 60), (2048, 3), (2049, 3), (2049, 90)])
+def test_leaf_eval_lists_equals_rows_given(T, ply):
+    """Leaf evaluation from the lists on both sides of its first launch's limit
+    (2,048 leaves) and with few and many successor rows (feature rows, unit
+    records), against the network over the features given as rows: the same
+    float32 operands, so 1e-5 bounds the sums' orders."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(4)
+    st = hive_gpu.random_positions(T, 7, ply, 11)[0]
+    mv, n, feat = ext.generate_legal_moves_and_fnn_features_batch(st, T)
+    got = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
+    rows, leaf = ext.fnn_list_successor_features_batch(st, mv, n, T)
+    off = torch.cumsum(n.to(torch.int64), 0) - n
+    want = ext.fnn_leaf_eval(torch.cat([feat, rows]), T, off, n, leaf, net)
+    for a, b in zip(got, want):
+        assert float((a - b).abs().max()) < 1e-5

@@ -1031,14 +1031,16 @@ HW_INL bool successor_range(SuccBoard& G, const SuccTables& K, const uint8_t* __
         }
         // -- units: a row starts one unless it places another common type on
         // the cell of the row before (a queen, mosquito or pillbug changes more
-        // than its class's counters, and a mosquito takes its neighbours' types)
+        // than its class's counters, and a mosquito takes its neighbours' types).
+        // A type that is not in hand starts one of its own, which units_pass marks
         uint32_t head[2];
         uint32_t last_to = ~0u;
+        const uint32_t mover = G.P.turn & 1;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const uint32_t pt = tp[j] >> 8, w = (uint32_t)(G.R.mosq - (int)to[j] + 23);
             const bool plain = (tp[j] & 0xFFu) == MV_PLACE && to[j] < (uint32_t)kCells && pt < 8 && ((0xBCu >> pt) & 1u) &&
-                               !K.dir[w < 47u ? w : 47u];
+                               ((G.R.hand >> (2u * (((pt - 1u) * 2u + mover) & 15u))) & 3u) && !K.dir[w < 47u ? w : 47u];
             const uint32_t share = plain ? to[j] : 0xFFFFu;  // rows of one unit carry the same cell
             const uint32_t up = grp_shfl(share, (l + kW - 1) & (kW - 1), lane);
             const uint32_t prev = l == 0 ? last_to : up;

@@ -292,6 +292,49 @@ def test_emulated_successor_units_any_rows(emu, oracle):
                             np.nonzero(got[r] != want[r])[0].tolist()) for r in bad[:6]]
 
 
+def _placements_on_shared_cells(st, beside_pillbug):
+    """Lists of consecutive placements on one cell: all eight types upwards,
+    then downwards, on empty cells next to the hive -- those beside a pillbug
+    of the player not placing, or the others."""
+    B = len(st)
+    mv = np.zeros((B, 256, 6), np.uint8)
+    roots, idx = [], []
+    h = st[:, 2645:2645 + 529]
+    for i in range(B):
+        occ = np.nonzero(h[i])[0]
+        me = int(st[i, 3412]) & 1
+        nb = lambda c: [c + d for d in (-23, -22, -1, 1, 22, 23) if 0 <= c + d < 529 and abs((c + d) % 23 - c % 23) < 2]
+        top = {int(c): int(st[i, (int(h[i][c]) - 1) * 529 + int(c)]) for c in occ}
+        pill = {c for c, t in top.items() if (t & 15) == 8 and ((t >> 4) & 1) != me}
+        near = sorted({x for c in top for x in nb(c) if h[i][x] == 0})
+        cells = [c for c in near if any(x in pill for x in nb(c)) == beside_pillbug][:2]
+        for k, c in enumerate(cells):
+            for j, t in enumerate([*range(1, 9), *range(8, 0, -1)]):
+                mv[i, 16 * k + j] = [0, t, 0, 0, int(c) & 255, int(c) >> 8]
+        roots += [i] * (16 * len(cells))
+        idx += range(16 * len(cells))
+    return mv, np.array(roots, np.int64), np.array(idx, np.int64)
+
+
+@pytest.mark.parametrize("beside_pillbug,mask,max_ply", [(False, 0, 30), (False, 7, 70)])
+def test_emulated_successor_units_shared_cell(emu, oracle, beside_pillbug, mask, max_ply):
+    """Placements of held and unheld types in a row on one cell, which join a
+    unit only where they share everything but their class's counters, against
+    the row-by-row program."""
+    st, _ = oracle.generate_positions(6, mask, max_ply, 31)
+    st = np.ascontiguousarray(st)
+    mv, roots, idx = _placements_on_shared_cells(st, beside_pillbug)
+    held = st[roots, 3395 + 8 * (st[roots, 3412] & 1).astype(int) + mv[roots, idx, 1]] > 0
+    assert len(roots) >= 64 and held.any() and not held.all()
+    want = np.full((len(roots), 122), np.nan, np.float32)
+    emu.emu_successor_rows(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
+                           ctypes.c_int64(st.shape[0]), _p(want))
+    for records in (False, True):
+        got = _units(emu, st, mv, roots, idx, 70, records)
+        bad = np.nonzero((got.view(np.uint32) != want.view(np.uint32)).any(1))[0]
+        assert len(bad) == 0, (records, [(int(roots[r]), mv[roots[r], idx[r]].tolist()) for r in bad[:6]])
+
+
 @pytest.mark.parametrize("flags,cap", [((1, 1, 1), 0), ((0, 0, 1), 0), ((1, 1, 1), 3)])
 def test_emulated_root_tactical_probe(emu, flags, cap):
     """hive_probe.hpp's group programs, orchestrated as hive_probe.hip's

@@ -81,6 +81,7 @@ struct SuccRoot {
                        // stacks (what a leaving top reveals), mosquitoes and pillbugs
     uint32_t cnt, hand, dn;  // 2-bit fields of the root (Unit)
     int mosq;          // cell of the next player's mosquito on top of a single-piece cell, else kNone
+    int pill;          // cell of its pillbug on top, else kNone
     int rlo, rhi;      // grid rows of the hive (empty board: the first move's row)
     uint8_t covered;   // a board this program covers
     uint8_t border;    // an occupied cell on the grid's border
@@ -177,7 +178,7 @@ HW_INL void succ_root(SuccBoard& G, const uint8_t* __restrict__ S, int lane, boo
         R.rlo = rows ? __ffs(rows) - 1 : kGrid / 2;
         R.rhi = rows ? 31 - __clz(rows) : kGrid / 2;
         build_rings(G, lane, R.rlo, R.rhi);
-        bool bad = false, single = false, mp = false, mine = false, own = false;
+        bool bad = false, single = false, mp = false, mine = false, own = false, bug = false;
         uint32_t cover = 0;
         int c = 0;
         if (l < n) {
@@ -188,6 +189,7 @@ HW_INL void succ_root(SuccBoard& G, const uint8_t* __restrict__ S, int lane, boo
             mp = pt == PT_M || pt == PT_P;
             own = col == next;
             mine = pt == PT_M && own && single;
+            bug = pt == PT_P && own;
             if (!bad) {
                 const int cls = (pt - 1) * 2 + col, q = P.queen[col ^ 1];
                 atomicOr(&G.vert[cls], 1u << l);
@@ -207,8 +209,9 @@ HW_INL void succ_root(SuccBoard& G, const uint8_t* __restrict__ S, int lane, boo
         R.cov[0] = grp_ballot(cover & 1u, lane);
         R.cov[1] = grp_ballot((cover >> 1) & 1u, lane);
         R.visit = grp_ballot(mp || own, lane) | R.tall;
-        const uint32_t mm = grp_ballot(mine, lane);
+        const uint32_t mm = grp_ballot(mine, lane), pb = grp_ballot(bug, lane);
         R.mosq = mm ? P.occ_cells[__ffs(mm) - 1] : kNone;
+        R.pill = pb ? P.occ_cells[__ffs(pb) - 1] : kNone;
         R.border = grp_ballot(l < 18 && (P.occ[l + 1] & kEdgeMask.m[l]) != 0u, lane) != 0;
         auto queen_ok = [&](int q) { return q == 0xFFFF || q < kCells; };
         const int turn = (P.turn + 1) & 0xFFFF;
@@ -1031,16 +1034,19 @@ HW_INL bool successor_range(SuccBoard& G, const SuccTables& K, const uint8_t* __
         }
         // -- units: a row starts one unless it places another common type on
         // the cell of the row before (a queen, mosquito or pillbug changes more
-        // than its class's counters, and a mosquito takes its neighbours' types).
-        // A type that is not in hand starts one of its own, which units_pass marks
+        // than its class's counters, a mosquito takes its neighbours' types, and a
+        // pillbug that throws the placed piece lets its class move).  A type that
+        // is not in hand starts one of its own, which units_pass marks
         uint32_t head[2];
         uint32_t last_to = ~0u;
         const uint32_t mover = G.P.turn & 1;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const uint32_t pt = tp[j] >> 8, w = (uint32_t)(G.R.mosq - (int)to[j] + 23);
+            const uint32_t pt = tp[j] >> 8;
+            const uint32_t w = (uint32_t)(G.R.mosq - (int)to[j] + 23), b = (uint32_t)(G.R.pill - (int)to[j] + 23);
             const bool plain = (tp[j] & 0xFFu) == MV_PLACE && to[j] < (uint32_t)kCells && pt < 8 && ((0xBCu >> pt) & 1u) &&
-                               ((G.R.hand >> (2u * (((pt - 1u) * 2u + mover) & 15u))) & 3u) && !K.dir[w < 47u ? w : 47u];
+                               ((G.R.hand >> (2u * (((pt - 1u) * 2u + mover) & 15u))) & 3u) && !K.dir[w < 47u ? w : 47u] &&
+                               !K.dir[b < 47u ? b : 47u];
             const uint32_t share = plain ? to[j] : 0xFFFFu;  // rows of one unit carry the same cell
             const uint32_t up = grp_shfl(share, (l + kW - 1) & (kW - 1), lane);
             const uint32_t prev = l == 0 ? last_to : up;

@@ -213,7 +213,8 @@ HW_INL void succ_root(SuccBoard& G, const uint8_t* __restrict__ S, int lane, boo
         R.mosq = mm ? P.occ_cells[__ffs(mm) - 1] : kNone;
         R.pill = pb ? P.occ_cells[__ffs(pb) - 1] : kNone;
         R.border = grp_ballot(l < 18 && (P.occ[l + 1] & kEdgeMask.m[l]) != 0u, lane) != 0;
-        auto queen_ok = [&](int q) { return q == 0xFFFF || q < kCells; };
+        // a recorded queen stands on the hive: the ring bytes reach no further than the hive's rows and two more
+        auto queen_ok = [&](int q) { return q == 0xFFFF || (q < kCells && pb_get(P.occ, q)); };
         const int turn = (P.turn + 1) & 0xFFFF;
         bad |= n > kArtN || P.result != 0 || turn == 0 || !queen_ok(P.queen[0]) || !queen_ok(P.queen[1]);
         R.queen_down = (P.qplaced >> next) & 1;

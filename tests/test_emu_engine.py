@@ -335,6 +335,30 @@ def test_emulated_successor_units_shared_cell(emu, oracle, beside_pillbug, mask,
         assert len(bad) == 0, (records, [(int(roots[r]), mv[roots[r], idx[r]].tolist()) for r in bad[:6]])
 
 
+@pytest.mark.parametrize("colour", [0, 1])
+def test_emulated_successor_units_queen_off_hive(emu, oracle, colour):
+    """Boards whose recorded queen cell is empty, near the hive and far from it,
+    give what the row-by-row program gives (the LDS starts with arbitrary
+    contents, so a read past the root's own tables shows)."""
+    st, _ = oracle.generate_positions(8, 0, 60, 41)
+    st = np.ascontiguousarray(st)
+    mv, n, _, _ = oracle.batch_legal_features_actions(st)
+    mv = np.ascontiguousarray(mv)
+    roots, idx = _all_rows(np.minimum(n, 12))
+    rng = np.random.default_rng(colour)
+    for i, s in enumerate(st):
+        free = np.nonzero(s[2645:2645 + 529] == 0)[0]
+        q = int(rng.choice(free)) if i % 2 else int(free[0 if i % 4 else -1])
+        s[3392 + 2 * colour: 3394 + 2 * colour] = [q & 255, q >> 8]
+        s[3414] |= 1 << colour
+    want = np.full((len(roots), 122), np.nan, np.float32)
+    emu.emu_successor_rows(_p(st), _p(mv), _p(roots), _p(idx), ctypes.c_int64(len(roots)),
+                           ctypes.c_int64(st.shape[0]), _p(want))
+    for records in (False, True):
+        got = _units(emu, st, mv, roots, idx, 30, records)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), records
+
+
 @pytest.mark.parametrize("flags,cap", [((1, 1, 1), 0), ((0, 0, 1), 0), ((1, 1, 1), 3)])
 def test_emulated_root_tactical_probe(emu, flags, cap):
     """hive_probe.hpp's group programs, orchestrated as hive_probe.hip's

@@ -198,8 +198,19 @@ __device__ __attribute__((aligned(16))) const uint8_t kZeroRow[kStateBytes] = {}
 // that lets that many run (4 waves per SIMD).
 constexpr int64_t kSuccGrid = 256 * 16;
 constexpr int kSuccWaves = 4;
-// rows per block: a kSuccSpread-th of the batch, from kSuccShort to kSuccBlock
+// rows per block: kSuccShort, or up to kSuccBlock while there are kSuccSpread blocks
 constexpr int kSuccShort = 8, kSuccBlock = 32, kSuccSpread = 2048;
+static_assert(kSuccBlock == kW, "a block lies in one window of successor_short_runs");
+// the row-by-row kernel: workgroups, and its register budget by index type --
+// the 32-bit row arithmetic fits 6 waves per SIMD (80 VGPRs, no spills; 24
+// workgroups' boards fill a CU's LDS), the 64-bit one 5 (96 VGPRs)
+constexpr int64_t kSingleGrid = 16384;
+// hg_fnn_successor_features' batches of at most this many rows are all its
+// work.  Row by row / by passes, us, base game and every piece: 17 K rows 26 / 57
+// and 42 / 83, 40 K 52 / 71 and 83 / 111, 107 K 146 / 95 and 233 / 143
+constexpr int64_t kSingleRows = 49152;
+template <typename Ix>
+constexpr int kSingleWaves = sizeof(Ix) == 4 ? 6 : 5;
 // lane groups a batch of leaves is spread over by cutting its lists into parts
 constexpr int kSuccParts = 8, kSuccTarget = 8192;
 
@@ -223,6 +234,21 @@ inline bool successor_narrow(int64_t rows_cap, int64_t num_roots) {
            num_roots <= ((int64_t)1 << 32) / kStateBytes && num_roots <= ((int64_t)1 << 32) / (kMaxLegal * 6);
 }
 
+// Rows in any order come to k_successor_features and k_successor_single in
+// windows of kW rows, which are the former's work if their runs of one root are
+// kSuccRun rows long on average: a pass costs as much as about that many rows
+// of the row-by-row program.
+constexpr int kSuccRun = 5;
+template <typename Ix>
+HW_INL bool successor_short_runs(const int64_t* __restrict__ a2r, Ix row, Ix N, int lane) {  // of the window of row
+    const int l = gl(lane);
+    const Ix i = row / (Ix)kW * (Ix)kW + (Ix)l;
+    const int64_t root = i < N ? a2r[i] : -1;
+    const int64_t before = grp_shfl(root, (l + kW - 1) & (kW - 1), lane);
+    const uint32_t live = grp_ballot(i < N, lane), runs = grp_ballot(i < N && (l == 0 || root != before), lane);
+    return __popc(live) < kSuccRun * __popc(runs);
+}
+
 // fnn_successor_features_kernel (game_logic.cu:182-229) over rows in any
 // order: the batch in blocks of rows, one per lane group in turn.  A block
 // works out the children of each root it meets together, so longer blocks
@@ -239,37 +265,59 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))
     load_succ_tables(K);
     const int lane = threadIdx.x, grp = lane >> 5;
     const Ix N = (Ix)n_rows, groups = (Ix)kPosPerWave * (Ix)gridDim.x;
-    Ix R = N / (Ix)kSuccSpread;
-    R = R < (Ix)kSuccShort ? (Ix)kSuccShort : (R > (Ix)kSuccBlock ? (Ix)kSuccBlock : R);
+    Ix R = (Ix)kSuccShort;  // a window's whole, half or quarter
+    while (R < (Ix)kSuccBlock && 2 * R <= N / (Ix)kSuccSpread) R *= 2;
     const Ix blocks = (N + R - 1) / R;
-    auto range = [&](Ix p, Ix& lo, Ix& hi) {
+    Ix lo = 0, hi = 0;
+    auto range = [&](Ix p) {
         const Ix q = p + (Ix)grp;
         lo = q * R < N ? q * R : N;
         hi = lo + R < N ? lo + R : N;
+        if (successor_short_runs<Ix>(a2r, lo, N, lane)) lo = hi;
     };
-    bool marks = true;
-    const bool every = N <= (Ix)kSuccStream;
-    Ix lo = 0, hi = 0;
-    if (every) {
-        const Ix per = (N + groups - 1) / groups;
-        lo = ((Ix)kPosPerWave * (Ix)blockIdx.x + (Ix)grp) * per;
-        lo = lo < N ? lo : N;
-        hi = lo + per < N ? lo + per : N;
-    } else {
-        bool general = false;
-        for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < blocks; p += groups) {
-            range(p, lo, hi);
-            general |= successor_range<Ix>(GS[grp], K, states, legal, MapRows{a2r, midx}, lo, hi, num_roots, kZeroRow,
-                                           lane, FeatureRows{feat_out});
-        }
-        __syncthreads();  // the marks, read by other lanes
-        marks = hw_wave_any(general);
+    bool general = false;
+    for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < blocks; p += groups) {
+        range(p);
+        if (!hw_wave_any(lo < hi)) continue;
+        general |= successor_range<Ix>(GS[grp], K, states, legal, MapRows{a2r, midx}, lo, hi, num_roots, kZeroRow, lane,
+                                       FeatureRows{feat_out});
     }
-    if (!marks) return;
-    for (Ix p = (Ix)kPosPerWave * blockIdx.x; every || p < blocks; p += groups) {
-        if (!every) range(p, lo, hi);
-        general_range<Ix>(GS[grp], states, legal, a2r, midx, lo, hi, num_roots, kZeroRow, lane, feat_out, every);
-        if (every) break;
+    __syncthreads();  // the marks, read by other lanes
+    if (!hw_wave_any(general)) return;
+    for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < blocks; p += groups) {
+        range(p);
+        general_range<Ix>(GS[grp], states, legal, a2r, midx, lo, hi, num_roots, kZeroRow, lane, feat_out);
+    }
+}
+
+// The same rows one at a time (successor_row): every row, or those of the
+// windows of short runs.  Lane group q of the grid takes pieces q,
+// q + 2 gridDim.x, ... of at most kSuccShort rows, a piece's rows as one
+// stream; one row each while the rows are few -- a short batch is bound by the
+// latency of each group's rows in series.
+// One move of each of 62 K roots 88 us (a pass for each 634 us), 107 K rows of
+// runs of four 135 us (201 us), shuffled 146 us (673 us).
+template <typename Ix>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSingleWaves<Ix>))) void k_successor_single(
+    const uint8_t* __restrict__ states, const uint8_t* __restrict__ legal, const int64_t* __restrict__ a2r,
+    const int64_t* __restrict__ midx, int64_t n_rows, int64_t num_roots, float* __restrict__ feat_out, int every) {
+    __shared__ Pos PS[kPosPerWave];
+    const int grp = threadIdx.x >> 5;
+    const Ix N = (Ix)n_rows, groups = (Ix)kPosPerWave * (Ix)gridDim.x;
+    int R = 1;  // divides a window
+    while (R < kSuccShort && (Ix)R * groups < N) R *= 2;
+    const Ix pieces = (N + R - 1) / R;
+    SuccessorStream st;
+    for (Ix p = (Ix)kPosPerWave * blockIdx.x; p < pieces; p += groups) {
+        Ix at = (p + (Ix)grp) * R;
+        if (!every) {
+            at = at < N ? at : N;
+            if (!successor_short_runs<Ix>(a2r, at, N, threadIdx.x)) at = N;
+            if (!hw_wave_any(at < N)) continue;
+        }
+        for (int k = 0; k < R; k++)
+            successor_row<Ix>(PS[grp], st, states, legal, a2r, midx, at < N ? at + (Ix)k : N, N, num_roots, kZeroRow,
+                              hw_opaque(threadIdx.x), feat_out);
     }
 }
 
@@ -890,15 +938,26 @@ int hg_fnn_successor_features(const uint8_t* states, const uint8_t* legal_moves,
                               const int64_t* action_to_root, const int64_t* move_indices, int64_t N, float* features,
                               void* stream) {
     if (N <= 0) return 0;
-    const int64_t each = N <= kSuccStream ? kPosPerWave : kSuccShort * kPosPerWave;
-    const int64_t pairs = (N + each - 1) / each;
-    const dim3 grid((unsigned)(pairs < kSuccGrid ? pairs : kSuccGrid));
-    if (successor_narrow(N, num_roots))
-        hipLaunchKernelGGL(k_successor_features<uint32_t>, grid, dim3(64), 0, (hipStream_t)stream, states, legal_moves,
-                           action_to_root, move_indices, N, num_roots, features);
-    else
-        hipLaunchKernelGGL(k_successor_features<int64_t>, grid, dim3(64), 0, (hipStream_t)stream, states, legal_moves,
-                           action_to_root, move_indices, N, num_roots, features);
+    hipStream_t s = (hipStream_t)stream;
+    const bool narrow = successor_narrow(N, num_roots), every = N <= kSingleRows;
+    if (!every) {  // long runs of a root's rows
+        const int64_t pairs = (N + kSuccShort * kPosPerWave - 1) / (kSuccShort * kPosPerWave);
+        const dim3 grid((unsigned)(pairs < kSuccGrid ? pairs : kSuccGrid));
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, states, legal_moves, action_to_root, move_indices, N,
+                               num_roots, features);
+        };
+        if (narrow) launch(k_successor_features<uint32_t>);
+        else launch(k_successor_features<int64_t>);
+    }
+    const int64_t pairs = (N + kPosPerWave - 1) / kPosPerWave;
+    const dim3 grid((unsigned)(pairs < kSingleGrid ? pairs : kSingleGrid));
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, states, legal_moves, action_to_root, move_indices, N, num_roots,
+                           features, every ? 1 : 0);
+    };
+    if (narrow) launch(k_successor_single<uint32_t>);
+    else launch(k_successor_single<int64_t>);
     return finish();
 }
 

@@ -393,3 +393,48 @@ def test_successor_rows_both_programs(ext, oracle, mask, rows):
     got = ext.fnn_successor_features_batch(torch.from_numpy(st).cuda(), torch.from_numpy(mv).cuda(),
                                            torch.from_numpy(roots).cuda(), torch.from_numpy(idx).cuda(), rows)
     assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("mask,rows", [(0, 49152), (0, 49153), (7, 60001)])
+def test_successor_rows_by_run_length(ext, oracle, mask, rows):
+    """Successor features on both sides of the batch size from which windows of
+    long runs of a root's rows are worked out by passes (49,152): whole lists,
+    single rows, runs about the line between the two programs, and rows out of
+    range, in stretches that start inside a window, against the oracle; moves
+    of no game among them, against the same rows in small batches."""
+    st, _ = oracle.generate_positions(300, mask, 120, 4200 + mask)
+    mv, n, _, _ = oracle.batch_legal_features_actions(st)
+    mv = np.array(mv)
+    whole = np.concatenate([np.full(int(k), i, np.int64) for i, k in enumerate(n)])
+    slot = np.concatenate([np.arange(int(k), dtype=np.int64) for k in n])
+    rng = np.random.default_rng(rows)
+    parts = []
+    while sum(len(r) for r, _ in parts) < rows:
+        kind, k = int(rng.integers(0, 4)), int(rng.integers(3, 8))
+        if kind == 0:  # a stretch of whole lists
+            a = int(rng.integers(0, len(whole) - 900))
+            parts.append((whole[a: a + 900], slot[a: a + 900]))
+        elif kind == 1:  # single rows
+            j = rng.integers(0, len(whole), 333)
+            parts.append((whole[j], slot[j]))
+        elif kind == 2:  # runs of k rows
+            r = rng.choice(np.nonzero(n >= k)[0], 60)
+            parts.append((np.repeat(r, k), np.tile(np.arange(k), 60)))
+        else:  # no root or slot
+            parts.append((np.full(21, len(st)), np.zeros(21, np.int64)))
+    roots = np.concatenate([r for r, _ in parts])[:rows].astype(np.int64)
+    idx = np.concatenate([i for _, i in parts])[:rows].astype(np.int64)
+    want = oracle.batch_successor_features(st, mv, np.minimum(roots, len(st) - 1), idx)
+    want[roots == len(st)] = 0.0
+
+    def features(m, r, i):
+        return ext.fnn_successor_features_batch(torch.from_numpy(st).cuda(), torch.from_numpy(m).cuda(),
+                                                torch.from_numpy(r).cuda(), torch.from_numpy(i).cuda(),
+                                                len(r)).cpu().numpy().view(np.uint32)
+
+    assert np.array_equal(features(mv, roots, idx), want.view(np.uint32))
+    odd = rng.choice(len(whole), 600, replace=False)
+    mv[whole[odd], slot[odd], 1] = rng.integers(0, 12, 600)  # other piece types, mostly not in hand
+    mv[whole[odd[::3]], slot[odd[::3]], 0] = 0
+    small = np.concatenate([features(mv, roots[a: a + 9000], idx[a: a + 9000]) for a in range(0, rows, 9000)])
+    assert np.array_equal(features(mv, roots, idx), small)

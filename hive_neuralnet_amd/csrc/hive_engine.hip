@@ -767,7 +767,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))
     bool marks = true, every = false, ready = false;
     Ix lo = 0, hi = 0;
     const Ix N = (Ix)offsets[T];
-    if (N <= (Ix)kSuccStream) {  // rows dealt to the lane groups, one or two each
+    if (!leaf_units((int64_t)N, T)) {  // rows dealt to the lane groups
         const Ix groups = (Ix)kPosPerWave * (Ix)gridDim.x, per = (N + groups - 1) / groups;
         lo = ((Ix)kPosPerWave * (Ix)blockIdx.x + (Ix)grp) * per;
         lo = lo < N ? lo : N;

@@ -294,7 +294,7 @@ __device__ __forceinline__ f4 vec4(const MlpLds& L, int which, int t, int g) {
 // kRoot: R[rows][64] <- Wr e + b_a1, value[rows] <- tanh(wv . e + bv).
 // !kRoot: row -> leaf = succ_leaf[row]; value[rows] <- tanh(wv . e + bv),
 //         logit[rows] <- wa2 . sigmoid(Ws e + R[leaf]) + ba2; with `units`
-//         and more than kSuccStream rows the features come from the rows' unit
+//         and rows enough (leaf_units) the features come from the rows' unit
 //         records (X holds the rows marked kRowGeneral only).
 template <bool kRoot>
 __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t blocks, const float* __restrict__ X, int64_t rows, int F,
@@ -412,7 +412,7 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
         f4 acc[4];  // every layer's sums start from its bias
 #pragma unroll
         for (int t = 0; t < 4; t++) acc[t] = vec4(L, kB1, t, g);
-        const bool packed = !kRoot && units && rows > hw::kSuccStream;
+        const bool packed = !kRoot && units && hw::leaf_units(rows, T);
         if (packed) {
             const uint32_t w = ok ? info[row] : 0u;
             if (w & hw::kRowGeneral) {

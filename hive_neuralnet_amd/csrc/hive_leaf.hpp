@@ -81,12 +81,14 @@ inline RowsPlan rows_plan_of(void* workspace, int64_t T) {
     return RowsPlan{o, o + T, o + T + 1, o + T + 1 + T * kMaxLegal};
 }
 
-// Batches of at most kSuccStream rows go row by row, a lane group each
-// (successor_row): one row takes about a third of a pass's time.  Leaf
-// evaluation by rows / by passes, us: mid-game base game 14 K rows 61 / 65,
+// Lists are worked out by passes where the batch has more rows than fit the
+// chip one at a time and its lists are not short, else row by row, a lane group
+// each (successor_row): one row takes about a third of a pass's time.
+// Leaf evaluation by rows / by passes, us: mid-game base game 14 K rows 61 / 65,
 // 21 K 74 / 67, 53 K 124 / 77; every piece 14 K 81 / 92, 19 K 101 / 95, 38 K
-// 150 / 97
-constexpr int kSuccStream = 16384;
+// 150 / 97; 10,000 lists of two moves 72 / 85, of three 85 / 87, of four 103 / 90
+constexpr int kSuccStream = 16384, kSuccMean = 3;
+__host__ __device__ inline bool leaf_units(int64_t rows, int64_t T) { return rows > kSuccStream && rows >= kSuccMean * T; }
 
 // hive_engine.hip: the plan of more than kPlanLeaves leaves (offsets, then the
 // row map), and the successor features of the planned rows

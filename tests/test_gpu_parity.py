@@ -438,3 +438,29 @@ def test_successor_rows_by_run_length(ext, oracle, mask, rows):
     mv[whole[odd[::3]], slot[odd[::3]], 0] = 0
     small = np.concatenate([features(mv, roots[a: a + 9000], idx[a: a + 9000]) for a in range(0, rows, 9000)])
     assert np.array_equal(features(mv, roots, idx), small)
+
+
+@pytest.mark.parametrize("T,cut,passes", [(300, 256, False), (620, 256, True), (10000, 3, False), (10000, 4, True)])
+def test_successor_rows_lists_both_programs(ext, T, cut, passes):
+    """The successor rows of T leaves' lists -- few rows, many, and many in lists
+    of three moves at most (`passes`: more than 16,384 rows in lists of at least
+    three on average) -- by both list entries, against the same rows in small
+    batches of fnn_successor_features_batch."""
+    from hive_neuralnet_amd.hive_gpu import random_positions
+    st = random_positions(T, 0, 120, 17)[0]
+    mv, n = ext.generate_legal_moves_batch(st, T)
+    n = n.clamp(max=cut)
+    N = int(n.sum())
+    assert (N > 16384 and N >= 3 * T) == passes
+    feat, a2r = ext.fnn_list_successor_features_batch(st, mv, n, T)
+    assert feat.shape[0] == N
+    start = torch.cumsum(n, 0) - n
+    slot = torch.arange(N, device="cuda") - start[a2r]
+    want = torch.cat([ext.fnn_successor_features_batch(st, mv, a2r[a: a + 9000].contiguous(), slot[a: a + 9000].contiguous(),
+                                                       min(9000, N - a)) for a in range(0, N, 9000)])
+    assert torch.equal(feat.view(torch.int32), want.view(torch.int32))
+    ws = torch.zeros((int(ext._lib.hg_successor_rows_workspace(T)),), dtype=torch.uint8, device="cuda")
+    out = torch.full((T * 256, 122), -7.0, device="cuda")
+    assert ext._lib.hg_successor_rows(st.data_ptr(), mv.data_ptr(), n.data_ptr(), T, ws.data_ptr(), out.data_ptr(),
+                                      torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out[:N].view(torch.int32), want.view(torch.int32)) and bool((out[N:] == -7.0).all())

@@ -197,6 +197,10 @@ __device__ __attribute__((aligned(16))) const uint8_t kZeroRow[kStateBytes] = {}
 // CUs; 18 workgroups' LDS boards fill a CU's 160 KB) and the register budget
 // that lets that many run (4 waves per SIMD).
 constexpr int64_t kSuccGrid = 256 * 16;
+// ... and for lists row by row: one row for each lane group up to 32 K rows
+// (four times the workgroups that run at once: leaf evaluation of 120 leaves with
+// every piece 67 -> 57 us, of 180 68 -> 63; 300 of the base game 52 -> 52)
+constexpr int64_t kRowsGrid = 4 * kSuccGrid;
 constexpr int kSuccWaves = 4;
 // rows per block: kSuccShort, or up to kSuccBlock while there are kSuccSpread blocks
 constexpr int kSuccShort = 8, kSuccBlock = 32, kSuccSpread = 2048;
@@ -767,7 +771,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kSuccWaves))
     bool marks = true, every = false, ready = false;
     Ix lo = 0, hi = 0;
     const Ix N = (Ix)offsets[T];
-    if (!leaf_units((int64_t)N, T)) {  // rows dealt to the lane groups
+    const bool passes = kToUnits<Out> ? leaf_units((int64_t)N, T) : list_units((int64_t)N, T);
+    if (!passes) {  // rows dealt to the lane groups
         const Ix groups = (Ix)kPosPerWave * (Ix)gridDim.x, per = (N + groups - 1) / groups;
         lo = ((Ix)kPosPerWave * (Ix)blockIdx.x + (Ix)grp) * per;
         lo = lo < N ? lo : N;
@@ -1034,7 +1039,7 @@ int successor_rows_after_plan(const uint8_t* states, const uint8_t* legal_moves,
     // every part of every leaf, and for a small batch a lane group per row (at
     // most 256 a leaf); workgroups with nothing to do end at once
     int64_t pairs = (T * successor_parts(T) + kPosPerWave - 1) / kPosPerWave;
-    const int64_t streams = T * kMaxLegal / kPosPerWave < kSuccGrid ? T * kMaxLegal / kPosPerWave : kSuccGrid;
+    const int64_t streams = T * kMaxLegal / kPosPerWave < kRowsGrid ? T * kMaxLegal / kPosPerWave : kRowsGrid;
     pairs = pairs < streams ? streams : pairs;
     const unsigned grid = (unsigned)(pairs < 16 * kSuccGrid ? pairs : 16 * kSuccGrid);
     const bool narrow = successor_narrow(T * kMaxLegal, T);  // at most 256 rows per leaf

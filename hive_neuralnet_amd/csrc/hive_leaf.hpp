@@ -89,6 +89,11 @@ inline RowsPlan rows_plan_of(void* workspace, int64_t T) {
 // 150 / 97; 10,000 lists of two moves 72 / 85, of three 85 / 87, of four 103 / 90
 constexpr int kSuccStream = 16384, kSuccMean = 3;
 __host__ __device__ inline bool leaf_units(int64_t rows, int64_t T) { return rows > kSuccStream && rows >= kSuccMean * T; }
+// The same where the rows' features are the result (a row's 488 bytes are
+// written either way).  By rows / by passes, plan included, us: base game 17 K
+// rows 40 / 45, every piece 19 K 60 / 74, 23 K 65 / 75
+constexpr int kListRows = 24576;
+__host__ __device__ inline bool list_units(int64_t rows, int64_t T) { return rows > kListRows && rows >= kSuccMean * T; }
 
 // hive_engine.hip: the plan of more than kPlanLeaves leaves (offsets, then the
 // row map), and the successor features of the planned rows

@@ -440,10 +440,11 @@ def test_successor_rows_by_run_length(ext, oracle, mask, rows):
     assert np.array_equal(features(mv, roots, idx), small)
 
 
-@pytest.mark.parametrize("T,cut,passes", [(300, 256, False), (620, 256, True), (10000, 3, False), (10000, 4, True)])
+@pytest.mark.parametrize("T,cut,passes", [(96, 256, False), (97, 256, False), (300, 256, False), (620, 256, True),
+                                          (10000, 3, False), (10000, 4, True)])
 def test_successor_rows_lists_both_programs(ext, T, cut, passes):
     """The successor rows of T leaves' lists -- few rows, many, and many in lists
-    of three moves at most (`passes`: more than 16,384 rows in lists of at least
+    of three moves at most (`passes`: more than 24,576 rows in lists of at least
     three on average) -- by both list entries, against the same rows in small
     batches of fnn_successor_features_batch."""
     from hive_neuralnet_amd.hive_gpu import random_positions
@@ -451,7 +452,7 @@ def test_successor_rows_lists_both_programs(ext, T, cut, passes):
     mv, n = ext.generate_legal_moves_batch(st, T)
     n = n.clamp(max=cut)
     N = int(n.sum())
-    assert (N > 16384 and N >= 3 * T) == passes
+    assert (N > 24576 and N >= 3 * T) == passes
     feat, a2r = ext.fnn_list_successor_features_batch(st, mv, n, T)
     assert feat.shape[0] == N
     start = torch.cumsum(n, 0) - n

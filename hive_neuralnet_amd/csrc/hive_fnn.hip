@@ -57,6 +57,9 @@
 // sum over the lane's 16 units plus two cross-lane steps (lanes l, l^16,
 // l^32, l^48 share a row).
 //
+// Rows that come out NaN are worked out again without the split
+// (leaf_plain_row): infinite operands have none.
+//
 // Floating point: everything between the products in fp32 with the reference's
 // operations (eps 1e-5, biased variance; sigmoid from the hardware exp2 /
 // reciprocal); summation orders differ from torch's GEMMs, so results agree
@@ -98,6 +101,7 @@ struct MlpLds {
     b8 w2[2][4][3][64];
     b8 w3[2][4][3][64];  // action_fc1 root half (root rows) or successor half (successor rows)
     float vec[7][kE];
+    float plain[kBlockWaves][kFMax];  // a row's inputs, per wave (leaf_plain_row)
 };
 enum { kB1, kLnW, kLnB, kB2, kWv, kWa2, kBa1 };
 
@@ -109,8 +113,6 @@ __device__ __forceinline__ void split3(f2 x, b2& p0, b2& p1, b2& p2) {
     p1 = __builtin_convertvector(r, b2);
     p2 = __builtin_convertvector(r - __builtin_convertvector(p1, f2), b2);
 }
-
-constexpr float kSplitMost = 3.38e38f;  // the largest bf16 is 3.39e38
 
 // The feature that fc1's step s takes at lane group g, element j: sections 0
 // and 2, 1 and 3, 4 and 5 (top pieces, next to the queen; hands, distances;
@@ -290,6 +292,52 @@ __device__ __forceinline__ f4 vec4(const MlpLds& L, int which, int t, int g) {
     return *reinterpret_cast<const f4*>(&L.vec[which][16 * t + 4 * g]);
 }
 
+__device__ __forceinline__ float wave_sum_f(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// A record's row (class k) into x, a quarter by each of four lanes; not inlined:
+// the MLP kernel that calls it once in a blue moon spilled 32 registers
+__device__ __attribute__((noinline)) void leaf_record_row(const hw::UnitRecord* __restrict__ rec, uint32_t k, int g,
+                                                          volatile float* x) {
+    float y[32];
+    hw::unit_slice(rec->u, g, rec->u.dsum[g], k, y);
+#pragma unroll
+    for (int p = 0; p < 32; p++) x[p < 24 ? 16 * (p >> 2) + 4 * g + (p & 3) : 96 + 8 * g + (p - 24)] = y[p];
+}
+
+// One row of the network without the split, a wave to it, a unit to each lane:
+// x (LDS) holds the row's features.  An infinite operand, or one that rounds
+// to a bf16 infinity (past 3.39e38), has no split -- its parts are NaN, and so
+// are the row's outputs -- but may have finite outputs.
+template <bool kRoot>
+__device__ __forceinline__ void leaf_plain_row(volatile float* x, int F, int u, const float* __restrict__ w1,
+                                               const float* __restrict__ b1, const float* __restrict__ lnw,
+                                               const float* __restrict__ lnb, const float* __restrict__ w2,
+                                               const float* __restrict__ b2, const float* __restrict__ wv, float bv,
+                                               const float* __restrict__ a1w, const float* __restrict__ a1b,
+                                               const float* __restrict__ a2w, float ba2, float* half, float& value,
+                                               float& logit) {
+    auto product = [&](const float* w, int n) {
+        float s = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < n; k++) s = __builtin_fmaf(w[k], x[k], s);
+        return s;
+    };
+    const float h = sigmoidf_(product(w1 + u * F, F) + b1[u]);
+    const float d = h - wave_sum_f(h) / (float)kE;
+    const float rstd = 1.0f / sqrtf(wave_sum_f(d * d) / (float)kE + 1e-5f);
+    x[u] = d * rstd * lnw[u] + lnb[u];
+    const float e = product(w2 + u * kE, kE) + b2[u];
+    value = tanhf(wave_sum_f(e * wv[u]) + bv);
+    x[u] = e;
+    const float r = product(a1w + u * 2 * kE + (kRoot ? 0 : kE), kE);
+    if constexpr (kRoot) half[u] = r + a1b[u];
+    else logit = wave_sum_f(sigmoidf_(r + half[u]) * a2w[u]) + ba2;
+}
+
 // X: [rows][F] features (F even, <= 128, 8-byte aligned rows).
 // kRoot: R[rows][64] <- Wr e + b_a1, value[rows] <- tanh(wv . e + bv).
 // !kRoot: row -> leaf = succ_leaf[row]; value[rows] <- tanh(wv . e + bv),
@@ -380,6 +428,7 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
     __syncthreads();
 
     const int lane = threadIdx.x & 63, g = lane >> 4;
+    bool odd = false;  // a row of the wave came out NaN
     for (int64_t tile = block + blocks * (threadIdx.x >> 6); tile < ntiles; tile += blocks * kBlockWaves) {
         // the weights are re-read from LDS in every tile: hoisted out of the
         // loop they would take hundreds of registers and leave one wave per SIMD
@@ -438,27 +487,12 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
             }
         } else {
             load_row();
-            // a feature past the parts' range (infinite, or rounding to it) has no
-            // split: its tile's first layer is summed plainly
-            float most = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 32; j += 2) most = fmaxf(fmaxf(most, fabsf(x[j])), fabsf(x[j + 1]));
-            if (__ballot(most > kSplitMost)) {
-                for (int k = 0; k < F; k++) {
-                    const float xk = ok ? X[row * F + k] : 0.0f;
+            for (int s = 0; s < 4; s++) {
+                b8 b[3];
+                split8([&](int j) { return x[8 * s + j]; }, b);
 #pragma unroll
-                    for (int t = 0; t < 4; t++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) acc[t][i] += w1[(16 * t + 4 * g + i) * F + k] * xk;
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    b8 b[3];
-                    split8([&](int j) { return x[8 * s + j]; }, b);
-#pragma unroll
-                    for (int t = 0; t < 4; t++) acc[t] = mfma3(L.w1[s][t], lane, b, acc[t]);
-                }
+                for (int t = 0; t < 4; t++) acc[t] = mfma3(L.w1[s][t], lane, b, acc[t]);
             }
         }
         if constexpr (!kRoot) {
@@ -530,6 +564,12 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
                     *reinterpret_cast<f4*>(R + row * kE + 16 * t + 4 * g) = h[t];
                 if (g == 0) value[row] = v;
             }
+            float all = v;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) all += h[t][i];
+            odd |= __ballot(ok && all != all) != 0;
         } else {
             float a = 0.0f;
 #pragma unroll
@@ -543,6 +583,36 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
                 value[row] = v;
                 logit[row] = a;
             }
+            odd |= __ballot(ok && (v != v || a != a)) != 0;
+        }
+    }
+    if (!odd) return;
+    __threadfence_block();  // the outputs, read by other lanes
+    const int u = hw_opaque(lane);
+    volatile float* const x = L.plain[threadIdx.x >> 6];
+    for (int64_t tile = block + blocks * (threadIdx.x >> 6); tile < ntiles; tile += blocks * kBlockWaves) {
+        for (int64_t row = tile * 16; row < rows && row < tile * 16 + 16; row++) {
+            float v = value[row], a = kRoot ? R[row * kE + u] : logit[row];
+            if (!__ballot(v != v || a != a)) continue;
+            bool record = false;
+            if constexpr (!kRoot) {
+                if (units && hw::leaf_units(rows, T)) {
+                    const uint32_t w = info[row];
+                    record = !(w & hw::kRowGeneral);
+                    if (record && u < 4) leaf_record_row(units + (row - (int64_t)(w & 255u)), (w >> 8) & 15u, u, x);
+                }
+            }
+            if (!record)
+                for (int k = u; k < F; k += 64) x[k] = X[row * F + k];
+            if constexpr (kRoot) {
+                leaf_plain_row<true>(x, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + row * kE, v, a);
+            } else {
+                int64_t leaf = succ_leaf[row];
+                leaf = leaf < 0 ? 0 : (leaf >= T ? T - 1 : leaf);
+                leaf_plain_row<false>(x, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + leaf * kE, v, a);
+                if (u == 0) logit[row] = a;
+            }
+            if (u == 0) value[row] = v;
         }
     }
 }
@@ -590,11 +660,6 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_first(
               a2w, pk, leaf_idx, vl_lens, stats);
 }
 
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 __device__ __forceinline__ float wave_max_f(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));

@@ -786,3 +786,52 @@ def test_leaf_eval_lists_equals_rows_given(T, ply):
     want = ext.fnn_leaf_eval(torch.cat([feat, rows]), T, off, n, leaf, net)
     for a, b in zip(got, want):
         assert float((a - b).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("what", ["infinite weight", "huge weight", "embedding overflow"])
+def test_leaf_eval_operands_without_split(what):
+    """Operands that no three bf16 parts add up to -- an infinite weight, a finite
+    one that rounds to a bf16 infinity, an embedding past float32 -- with finite
+    outputs: the network over rows given and over unit records against float64
+    (infinite or saturated units are 0 or 1, so the bound is that of 64 to 122
+    float32 terms a sum)."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(8)
+    with torch.no_grad():
+        if what == "infinite weight":
+            net.fc1.weight[3, 102] = float("inf")  # the feature of the turns left, never 0 here
+            net.fc1.weight[40, 102] = float("-inf")
+        elif what == "huge weight":
+            net.fc1.weight[3, 102] = 3.4e38
+        else:  # unit 7 of the embedding: 2 * 3.4e38
+            net.ln1.weight[0], net.ln1.bias[0] = 0.0, 2.0
+            net.fc2.weight[7, 0] = 3.4e38
+            net.action_fc1.weight[:, 64 + 7] = net.action_fc1.weight[:, 7]  # no infinity meets another sign's
+    T = 420
+    st = hive_gpu.random_positions(T, 0, 110, 23)[0]
+    mv, n, feat = ext.generate_legal_moves_and_fnn_features_batch(st, T)
+    rows, leaf = ext.fnn_list_successor_features_batch(st, mv, n, T)
+    N = rows.shape[0]
+    assert N > 16384
+    off = torch.cumsum(n.to(torch.int64), 0) - n
+    net64 = seeded_large(8).double()
+    net64.load_state_dict({k: v.double() for k, v in net.state_dict().items()})
+    with torch.no_grad():
+        e0, e1 = net64.encode(feat.double()), net64.encode(rows.double())
+        value, child = net64.value_head(e0).squeeze(1), -net64.value_head(e1).squeeze(1)
+        logit = net64.score_actions(e0[leaf], e1)
+    slot = torch.arange(N, device="cuda") - off[leaf]
+    dense = torch.full((T, 256), -float("inf"), dtype=torch.float64, device="cuda")
+    dense[leaf, slot] = logit
+    priors = torch.nan_to_num(torch.softmax(dense, 1), nan=0.0)
+    child_q = torch.zeros((T, 256), dtype=torch.float64, device="cuda")
+    child_q[leaf, slot] = child
+    assert bool(torch.isfinite(priors).all() and torch.isfinite(child_q).all())
+    for got in (ext.fnn_leaf_eval(torch.cat([feat, rows]), T, off, n, leaf, net),
+                ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)):
+        for a, b in zip(got, (priors, value, child_q)):
+            assert float((a.double() - b).abs().max()) < 1e-5

@@ -58,18 +58,18 @@ def build_forward_batch(ext, state_bytes: torch.Tensor, batch_size: int, num_act
     else:
         legal_moves, num_legal, root_features = ext.generate_legal_moves_and_fnn_features_batch(state_bytes, batch_size)
         num_actions = num_legal.to(torch.int64)
-    B = int(batch_size)
+    B, dev = int(batch_size), state_bytes.device
     counts = num_actions.clamp(0, legal_moves.shape[1])
-    if B > 0 and min(counts.shape[0], legal_moves.shape[0], state_bytes.numel() // hive_gpu.SIZEOF_HIVE_STATE) >= B:
+    roots = min(legal_moves.shape[0], state_bytes.numel() // hive_gpu.SIZEOF_HIVE_STATE)
+    if B > 0 and counts.shape == (B,) and roots >= B:
         # rows in (root, slot) order, planned on the device: one host read of the row count
         succ, action_to_root = ext.fnn_list_successor_features_batch(state_bytes, legal_moves, counts.to(torch.int32), B)
         return root_features, succ if succ.shape[0] else root_features[:0], action_to_root, num_actions
     # fewer roots than the batch names: the rows of the missing ones are zero
-    dev = state_bytes.device
     total = int(counts.sum().item())
-    action_to_root = torch.repeat_interleave(torch.arange(B, device=dev, dtype=torch.int64), counts, output_size=total)
     if total == 0:
-        return root_features, root_features[:0], action_to_root, num_actions
+        return root_features, root_features[:0], torch.zeros((0,), dtype=torch.int64, device=dev), num_actions
+    action_to_root = torch.repeat_interleave(torch.arange(B, device=dev, dtype=torch.int64), counts, output_size=total)
     starts = torch.cumsum(counts, 0) - counts
     move_indices = torch.arange(total, device=dev, dtype=torch.int64) - starts[action_to_root]
     succ = ext.fnn_successor_features_batch(state_bytes, legal_moves, action_to_root, move_indices, total)

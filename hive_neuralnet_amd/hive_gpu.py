@@ -429,7 +429,7 @@ class HiveGpuExtension:
         if N > 0:
             _check(self._lib.hg_successor_planned_rows(states.data_ptr(), legal_moves.data_ptr(), B, ws.data_ptr(),
                                                        feat.data_ptr(), _stream()), "successor_planned_rows")
-        return feat, ws[B + 1: B + 1 + N]
+        return feat, ws[B + 1: B + 1 + N].clone()  # not a view: it would keep the plan's 4 KB a root alive
 
     # ---- fused FNN leaf evaluation (no reference counterpart; see include/hive_gpu.h)
     def fnn_leaf_eval(self, features, T: int, offsets, num_legal, succ_leaf, net, head_biases=None):

@@ -28,6 +28,7 @@ def test_build_forward_batch_matches_oracle(oracle, mask, max_ply):
     want_a2r = np.repeat(np.arange(B), on)
     mi = np.concatenate([np.arange(k) for k in on])
     assert np.array_equal(_np(a2r), want_a2r)
+    assert a2r.untyped_storage().nbytes() == 8 * len(want_a2r)  # its own memory: the plan's is given back
     want_succ = oracle.batch_successor_features(st, om, want_a2r, mi)
     assert np.array_equal(_np(succ).view(np.uint32), want_succ.view(np.uint32))
     legal, nl, feat = ext.generate_legal_moves_and_fnn_features_batch(states, B)

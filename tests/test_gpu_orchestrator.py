@@ -737,9 +737,9 @@ def test_reserve_candidates_match_oracle(mask, max_ply, immobile):
 def test_leaf_eval_products_against_float64(T, each, scale):
     """The network's products (float32 operands in three bf16 parts) at tile
     edges and remainders, features from small to large and infinite or NaN
-    ones among them, against float64: the values and child Q of finite rows
-    within 1e-5 (64 to 122 float32 terms a sum, sigmoids in between), and the
-    rows of non-finite features non-finite where float64's are."""
+    ones among them, against float64: the values, child Q and priors of finite
+    rows within 1e-5 (64 to 122 float32 terms a sum, sigmoids in between), and
+    the rows of non-finite features non-finite where float64's are."""
     import torch
 
     from hive_neuralnet_amd import hive_gpu
@@ -756,22 +756,27 @@ def test_leaf_eval_products_against_float64(T, each, scale):
     n = torch.full((T,), each, dtype=torch.int32, device="cuda")
     off = torch.arange(T, device="cuda", dtype=torch.int64) * each
     leaf = torch.arange(T, device="cuda").repeat_interleave(each)
-    _, value, child_q = ext.fnn_leaf_eval(f, T, off, n, leaf, net)
+    priors, value, child_q = ext.fnn_leaf_eval(f, T, off, n, leaf, net)
     net64 = seeded_large(21).double()
     with torch.no_grad():
-        want = net64.value_head(net64.encode(f.double())).squeeze(1)
-    got = torch.cat([value, -child_q[:, :each].reshape(-1)]).double()
+        e = net64.encode(f.double())
+        want = torch.cat([net64.value_head(e).squeeze(1),
+                          torch.softmax(net64.score_actions(e[:T][leaf], e[T:]).view(T, each), 1).reshape(-1)])
+    got = torch.cat([value, -child_q[:, :each].reshape(-1), priors[:, :each].reshape(-1)]).double()
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     ok = torch.isfinite(want)
     assert float((got[ok] - want[ok]).abs().max()) < 1e-5
 
 
-@pytest.mark.parametrize("T,ply", [(1, 60), (2048, 3), (2049, 3), (2049, 90)])
-def test_leaf_eval_lists_equals_rows_given(T, ply):
+@pytest.mark.parametrize("T,ply,cut,total", [(1, 60, 256, None), (2048, 3, 7, None), (2049, 3, 7, None),
+                                             (2048, 3, 9, 16384), (2049, 3, 9, 16384), (2048, 3, 9, 16385),
+                                             (2049, 90, 256, None), (6000, 90, 4, 17999), (6000, 90, 4, 18000)])
+def test_leaf_eval_lists_equals_rows_given(T, ply, cut, total):
     """Leaf evaluation from the lists on both sides of its first launch's limit
-    (2,048 leaves) and with few and many successor rows (feature rows, unit
-    records), against the network over the features given as rows: the same
-    float32 operands, so 1e-5 bounds the sums' orders."""
+    (2,048 leaves) and of the rules by which the successors' features come as
+    rows or from unit records (more than 16,384 rows, lists of at least three
+    moves on average), against the network over the features given as rows:
+    the same operands in the same order, so the same bits."""
     import torch
 
     from hive_neuralnet_amd import hive_gpu
@@ -780,21 +785,82 @@ def test_leaf_eval_lists_equals_rows_given(T, ply):
     net = seeded_large(4)
     st = hive_gpu.random_positions(T, 7, ply, 11)[0]
     mv, n, feat = ext.generate_legal_moves_and_fnn_features_batch(st, T)
-    got = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
+    n = n.clamp(max=cut)
+    if total is not None:  # exactly so many rows
+        n[torch.nonzero(n)[: int(n.sum()) - total, 0]] -= 1
+        assert int(n.sum()) == total
     rows, leaf = ext.fnn_list_successor_features_batch(st, mv, n, T)
+    records = rows.shape[0] > 16384 and rows.shape[0] >= 3 * T
+    assert records == ((T, cut, total) in [(2048, 9, 16385), (2049, 256, None), (6000, 4, 18000)])
     off = torch.cumsum(n.to(torch.int64), 0) - n
+    got = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
     want = ext.fnn_leaf_eval(torch.cat([feat, rows]), T, off, n, leaf, net)
     for a, b in zip(got, want):
-        assert float((a - b).abs().max()) < 1e-5
+        assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("what", ["infinite weight", "huge weight", "embedding overflow"])
+def test_leaf_eval_lists_general_rows():
+    """Leaf evaluation of more than 16,384 rows with rows that the unit program
+    leaves to the row-by-row one (moves of no game, a board past the pieces of a
+    set, a finished game, a queen recorded off the hive): their features come as
+    rows among the unit records, and the outputs are those of the row-by-row
+    features to the bit.  The leaves' own features go through as they are."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(4)
+    T = 500
+    st = hive_gpu.random_positions(T, 7, 100, 12)[0]
+    mv, n, feat = ext.generate_legal_moves_and_fnn_features_batch(st, T)
+    off = torch.cumsum(n.to(torch.int64), 0) - n
+    leaf = torch.arange(T, device="cuda").repeat_interleave(n.to(torch.int64))
+    slot = torch.arange(leaf.shape[0], device="cuda") - off[leaf]
+    N = leaf.shape[0]
+    assert N > 16384
+    st[7, 3396:3404] = 9
+    st[60, 3415] = 1
+    st[61, 3392:3394] = 0  # white's queen recorded at cell 0
+    g = torch.Generator(device="cuda").manual_seed(5)
+    odd = torch.randperm(N, generator=g, device="cuda")[:900]
+    mv[leaf[odd], slot[odd], 1] = torch.randint(0, 12, (900,), generator=g, device="cuda", dtype=torch.uint8)
+    mv[leaf[odd[::3]], slot[odd[::3]], 0] = 0  # placements of types mostly not in hand
+    rows = torch.cat([ext.fnn_successor_features_batch(st, mv, leaf[a: a + 9000], slot[a: a + 9000].contiguous(),
+                                                       min(9000, N - a)) for a in range(0, N, 9000)])
+    got = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
+    want = ext.fnn_leaf_eval(torch.cat([feat, rows]), T, off, n, leaf, net)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_leaf_eval_lists_wide_offsets():
+    """137,519 leaves, whose feature offsets may pass 2^32: 64-bit row arithmetic
+    in the successor kernel, against the leaves evaluated in parts."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(4)
+    T, P = 137519, 4000
+    base = hive_gpu.random_positions(P, 0, 90, 13)[0]
+    bm, bn, bf = ext.generate_legal_moves_and_fnn_features_batch(base, P)
+    bn = bn.clamp(max=6)
+    take = torch.arange(T, device="cuda") % P
+    got = ext.fnn_leaf_eval_lists(base[take], bm[take], bn[take].contiguous(), bf[take], T, net)
+    want = ext.fnn_leaf_eval_lists(base, bm, bn, bf, P, net)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b[take])
+
+
+@pytest.mark.parametrize("what", ["any operand", "infinite weight", "huge weight", "embedding overflow"])
 def test_leaf_eval_operands_without_split(what):
-    """Operands that no three bf16 parts add up to -- an infinite weight, a finite
-    one that rounds to a bf16 infinity, an embedding past float32 -- with finite
-    outputs: the network over rows given and over unit records against float64
-    (infinite or saturated units are 0 or 1, so the bound is that of 64 to 122
-    float32 terms a sum)."""
+    """A network as it is drawn, then operands that no three bf16 parts add up to
+    -- an infinite weight, a finite one that rounds to a bf16 infinity, an
+    embedding past float32 -- with finite outputs: the network over rows given
+    and over unit records against float64 (infinite or saturated units are 0 or
+    1, so the bound is that of 64 to 122 float32 terms a sum)."""
     import torch
 
     from hive_neuralnet_amd import hive_gpu
@@ -807,7 +873,7 @@ def test_leaf_eval_operands_without_split(what):
             net.fc1.weight[40, 102] = float("-inf")
         elif what == "huge weight":
             net.fc1.weight[3, 102] = 3.4e38
-        else:  # unit 7 of the embedding: 2 * 3.4e38
+        elif what == "embedding overflow":  # unit 7 of the embedding: 2 * 3.4e38
             net.ln1.weight[0], net.ln1.bias[0] = 0.0, 2.0
             net.fc2.weight[7, 0] = 3.4e38
             net.action_fc1.weight[:, 64 + 7] = net.action_fc1.weight[:, 7]  # no infinity meets another sign's

@@ -14,9 +14,12 @@
 // are one *unit*: a lane works a unit out once, and the group then writes the
 // rows of each unit, adding the placed type's own contributions per row.
 //
-// What bounds it: VALU issue, as before.  426 K mid-game rows: successor_row
-// (about 300 VALU instructions a row) 439 us, here 136 us as features and 111 us
-// as the units' records.
+// What bounds it: VALU issue for half of the time (76 instructions a row of 427 K
+// mid-game rows: 127 K of a SIMD's 249 K cycles), and the passes' serial chains --
+// LDS round trips, floods, moves tried one after another -- which the 2.5 waves a
+// SIMD that are left on average do not cover; the longest lists end the launch.
+// 426 K mid-game rows: successor_row (about 300 VALU instructions a row) 439 us,
+// here 136 us as features and 111-114 us as the units' records.
 #pragma once
 
 #include "hive_phases.hpp"
@@ -213,8 +216,11 @@ HW_INL void succ_root(SuccBoard& G, const uint8_t* __restrict__ S, int lane, boo
         R.mosq = mm ? P.occ_cells[__ffs(mm) - 1] : kNone;
         R.pill = pb ? P.occ_cells[__ffs(pb) - 1] : kNone;
         R.border = grp_ballot(l < 18 && (P.occ[l + 1] & kEdgeMask.m[l]) != 0u, lane) != 0;
-        // a recorded queen stands on the hive: the ring bytes reach no further than the hive's rows and two more
-        auto queen_ok = [&](int q) { return q == 0xFFFF || (q < kCells && pb_get(P.occ, q)); };
+        // a recorded queen's cell is in the rows whose ring bytes are built: the hive's and two more each way
+        auto queen_ok = [&](int q) {
+            const int r = row_of(q);
+            return q == 0xFFFF || (q < kCells && r >= R.rlo - 2 && r <= R.rhi + 2);
+        };
         const int turn = (P.turn + 1) & 0xFFFF;
         bad |= n > kArtN || P.result != 0 || turn == 0 || !queen_ok(P.queen[0]) || !queen_ok(P.queen[1]);
         R.queen_down = (P.qplaced >> next) & 1;

@@ -22,20 +22,22 @@
 //                      zero beyond the legal count.
 //
 // The products run on the bf16 matrix cores at float32's accuracy: a float
-// is the exact sum of three bf16 parts (8 significant bits each), and of the
-// nine products of two such sums the six that reach 2^-26 of the whole are
-// taken, v_mfma_f32_16x16x32_bf16 each, accumulated in float32.  That is six
-// times the multiplications at sixteen times the rate of the fp32 matrix
-// instruction; what is left out is a quarter of a float32 rounding.  The
+// is the exact sum of three bf16 parts (8 significant bits each: the second is
+// at most 2^-9 of the first, the third 2^-18), and of the nine products of two
+// such sums the six down to 2^-18 of the whole are taken,
+// v_mfma_f32_16x16x32_bf16 each, accumulated in float32.  That is six times the
+// multiplications at sixteen times the rate of the fp32 matrix instruction;
+// what is left out is at most 2^-26, a quarter of a float32 rounding.  The
 // weights are split once per evaluation, the activations as they come.
 // Measured against the fp32 instruction (427 K successor rows): 143 -> 91 us,
 // 78 us with the units' records for features, the sums started from the biases
 // and fused multiply-adds around the products; the outputs' distance from
 // float64 is the same (1.4e-7 / 1.4e-7 to 8.5e-7 / 7.7e-7 relative over the seeds
-// tried).  Bound now by VALU issue (~750 a tile, a third of it the splits) and
-// the matrix pipe (168 instructions a tile), which add up to about the time
-// measured; not by the 96 KB of LDS reads a tile: two tiles per read took as
-// long (85.7 us against 85.9 before the multiply-adds).
+// tried).  Bound now by VALU issue (805 a tile besides the products, a third of
+// it the splits) and the matrix pipe (168 instructions a tile, 16 cycles each):
+// 84 K and 70 K of a SIMD's 171 K cycles, which add up; not by the 96 KB of LDS
+// reads a tile: two tiles per read took as long (85.7 us against 85.9 before
+// the multiply-adds).
 //
 // Matrix-core layout (16x16x32, D = A.B + C, A 16x32, B 32x16): lane l holds
 // A[l%16][8 (l/16) + j], B[8 (l/16) + j][l%16] (j < 8) and D[4(l/16)+i][l%16]
@@ -101,7 +103,6 @@ struct MlpLds {
     b8 w2[2][4][3][64];
     b8 w3[2][4][3][64];  // action_fc1 root half (root rows) or successor half (successor rows)
     float vec[7][kE];
-    float plain[kBlockWaves][kFMax];  // a row's inputs, per wave (leaf_plain_row)
 };
 enum { kB1, kLnW, kLnB, kB2, kWv, kWa2, kBa1 };
 
@@ -298,42 +299,44 @@ __device__ __forceinline__ float wave_sum_f(float v) {
     return v;
 }
 
-// A record's row (class k) into x, a quarter by each of four lanes; not inlined:
-// the MLP kernel that calls it once in a blue moon spilled 32 registers
-__device__ __attribute__((noinline)) void leaf_record_row(const hw::UnitRecord* __restrict__ rec, uint32_t k, int g,
-                                                          volatile float* x) {
-    float y[32];
+// Feature f of a record's row (class k), another for each lane; not inlined: the
+// MLP kernel, which calls it once in a blue moon, spilled 32 registers
+__device__ __attribute__((noinline)) float leaf_record_feature(const hw::UnitRecord* __restrict__ rec, uint32_t k, int f) {
+    const int g = f < 96 ? (f >> 2) & 3 : ((f - 96) >> 3) & 3, at = f < 96 ? 4 * (f >> 4) + (f & 3) : 24 + (f & 7);
+    float y[32], x = 0.0f;
     hw::unit_slice(rec->u, g, rec->u.dsum[g], k, y);
 #pragma unroll
-    for (int p = 0; p < 32; p++) x[p < 24 ? 16 * (p >> 2) + 4 * g + (p & 3) : 96 + 8 * g + (p - 24)] = y[p];
+    for (int p = 0; p < 32; p++) x = p == at ? y[p] : x;
+    return x;
 }
 
-// One row of the network without the split, a wave to it, a unit to each lane:
-// x (LDS) holds the row's features.  An infinite operand, or one that rounds
-// to a bf16 infinity (past 3.39e38), has no split -- its parts are NaN, and so
-// are the row's outputs -- but may have finite outputs.
+// One row of the network without the split, a wave to it, a unit to each lane
+// u, whose inputs are the features x0 = x[u], x1 = x[64 + u].  An infinite
+// operand, or one that rounds to a bf16 infinity (past 3.39e38), has no split
+// -- its parts are NaN, and so are the row's outputs -- but may have finite
+// outputs.
 template <bool kRoot>
-__device__ __forceinline__ void leaf_plain_row(volatile float* x, int F, int u, const float* __restrict__ w1,
+__device__ __forceinline__ void leaf_plain_row(float x0, float x1, int F, int u, const float* __restrict__ w1,
                                                const float* __restrict__ b1, const float* __restrict__ lnw,
                                                const float* __restrict__ lnb, const float* __restrict__ w2,
                                                const float* __restrict__ b2, const float* __restrict__ wv, float bv,
                                                const float* __restrict__ a1w, const float* __restrict__ a1b,
                                                const float* __restrict__ a2w, float ba2, float* half, float& value,
                                                float& logit) {
-    auto product = [&](const float* w, int n) {
-        float s = 0.0f;
+    auto product = [&](const float* w, float x, int n, float s) {  // s + w[0] x of lane 0 + ..
 #pragma unroll 1
-        for (int k = 0; k < n; k++) s = __builtin_fmaf(w[k], x[k], s);
+        for (int k = 0; k < n; k++)
+            s = __builtin_fmaf(w[k], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), k)), s);
         return s;
     };
-    const float h = sigmoidf_(product(w1 + u * F, F) + b1[u]);
+    float h = product(w1 + u * F, x0, F < 64 ? F : 64, 0.0f);
+    if (F > 64) h = product(w1 + u * F + 64, x1, F - 64, h);
+    h = sigmoidf_(h + b1[u]);
     const float d = h - wave_sum_f(h) / (float)kE;
     const float rstd = 1.0f / sqrtf(wave_sum_f(d * d) / (float)kE + 1e-5f);
-    x[u] = d * rstd * lnw[u] + lnb[u];
-    const float e = product(w2 + u * kE, kE) + b2[u];
+    const float e = product(w2 + u * kE, d * rstd * lnw[u] + lnb[u], kE, 0.0f) + b2[u];
     value = tanhf(wave_sum_f(e * wv[u]) + bv);
-    x[u] = e;
-    const float r = product(a1w + u * 2 * kE + (kRoot ? 0 : kE), kE);
+    const float r = product(a1w + u * 2 * kE + (kRoot ? 0 : kE), e, kE, 0.0f);
     if constexpr (kRoot) half[u] = r + a1b[u];
     else logit = wave_sum_f(sigmoidf_(r + half[u]) * a2w[u]) + ba2;
 }
@@ -589,27 +592,26 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
     if (!odd) return;
     __threadfence_block();  // the outputs, read by other lanes
     const int u = hw_opaque(lane);
-    volatile float* const x = L.plain[threadIdx.x >> 6];
     for (int64_t tile = block + blocks * (threadIdx.x >> 6); tile < ntiles; tile += blocks * kBlockWaves) {
         for (int64_t row = tile * 16; row < rows && row < tile * 16 + 16; row++) {
             float v = value[row], a = kRoot ? R[row * kE + u] : logit[row];
             if (!__ballot(v != v || a != a)) continue;
-            bool record = false;
+            const hw::UnitRecord* rec = nullptr;
+            uint32_t k = 0;
             if constexpr (!kRoot) {
-                if (units && hw::leaf_units(rows, T)) {
-                    const uint32_t w = info[row];
-                    record = !(w & hw::kRowGeneral);
-                    if (record && u < 4) leaf_record_row(units + (row - (int64_t)(w & 255u)), (w >> 8) & 15u, u, x);
+                if (units && hw::leaf_units(rows, T) && !(info[row] & hw::kRowGeneral)) {
+                    rec = units + (row - (int64_t)(info[row] & 255u));
+                    k = (info[row] >> 8) & 15u;
                 }
             }
-            if (!record)
-                for (int k = u; k < F; k += 64) x[k] = X[row * F + k];
+            const float x0 = rec ? leaf_record_feature(rec, k, u) : u < F ? X[row * F + u] : 0.0f;
+            const float x1 = rec ? leaf_record_feature(rec, k, 64 + u) : 64 + u < F ? X[row * F + 64 + u] : 0.0f;
             if constexpr (kRoot) {
-                leaf_plain_row<true>(x, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + row * kE, v, a);
+                leaf_plain_row<true>(x0, x1, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + row * kE, v, a);
             } else {
                 int64_t leaf = succ_leaf[row];
                 leaf = leaf < 0 ? 0 : (leaf >= T ? T - 1 : leaf);
-                leaf_plain_row<false>(x, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + leaf * kE, v, a);
+                leaf_plain_row<false>(x0, x1, F, u, w1, b1, lnw, lnb, w2, b2, wv, bv, a1w, a1b, a2w, ba2, R + leaf * kE, v, a);
                 if (u == 0) logit[row] = a;
             }
             if (u == 0) value[row] = v;
@@ -636,10 +638,11 @@ __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_mlp(const float* __re
 
 // The first launch of a short evaluation: k_leaf_prep's blocks (their first 256
 // threads) beside the root rows' tiles, whose blocks take the weights from the
-// network itself instead of waiting for the packed ones.  Every block fits the
-// chip at once (one per CU) up to kFirstLeaves leaves: 128 tile blocks, 81 of
-// packing, the plan's and the counters'.  Base-game leaf evaluation: 2,048 leaves
-// 83 us, 2,100 (the leaf rows' network in a launch of its own) 100 us.
+// network itself instead of waiting for the packed ones.  At kFirstLeaves leaves
+// every block has a CU of its own: 128 tile blocks, 81 of packing, the plan's and
+// the counters' (219 of 256; sizes between this one and where they no longer do,
+// about 2,580 leaves, were not tried).  Base-game leaf evaluation: 2,048 leaves 83
+// us, 2,100 (the leaf rows' network in a launch of its own) 100 us.
 constexpr int64_t kFirstLeaves = 2048;
 __global__ __launch_bounds__(64 * kBlockWaves) void k_leaf_first(
     int root_blocks, const float* __restrict__ X, int64_t T, int F, hw::RowsPlan plan, int plan_blocks,

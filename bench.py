@@ -336,7 +336,9 @@ def mcts_leg(args):
     sims = c["sims"]
     Lm = c["leaf_legal"] / max(1, sims)
     Dm = c["vl_len"] / max(1, sims)
-    b_sim = 5976 + 535 * Lm + 16 * Dm
+    # a child's 47 bytes in and out of the tree, its unit's record (64, shared by the rows of a
+    # placement cell) and its row's word
+    b_sim = 5976 + 115 * Lm + 16 * Dm
     value = sims / wall
     achieved = b_sim * value / 1e9
     out = {
@@ -356,7 +358,7 @@ def mcts_leg(args):
                                  if args.mcts_roots == "empty" and cfg.wave_parallel else None),
                      "traffic_is": "HBM bytes per simulation over the schedule's waves from the empty board, "
                                    "rocprofv3 FETCH_SIZE + WRITE_SIZE (profiles/mcts_c5_traffic.txt)",
-                     "bytes_per_sim": b_sim, "formula": "5976 + 535*L + 16*D"},
+                     "bytes_per_sim": b_sim, "formula": "5976 + 115*L + 16*D"},
     }
     if not args.no_cpu:
         threads = baseline_threads(args)

@@ -592,6 +592,13 @@ __device__ __forceinline__ void leaf_mlp(MlpLds& L, int64_t block, int64_t block
     if (!odd) return;
     __threadfence_block();  // the outputs, read by other lanes
     const int u = hw_opaque(lane);
+    // a NaN in the encoder itself is in every output of every row
+    bool lost = b1[u] != b1[u] || lnw[u] != lnw[u] || lnb[u] != lnb[u] || b2[u] != b2[u];
+#pragma unroll 1
+    for (int k = 0; k < F; k++) lost |= w1[u * F + k] != w1[u * F + k];
+#pragma unroll 1
+    for (int k = 0; k < kE; k++) lost |= w2[u * kE + k] != w2[u * kE + k];
+    if (__ballot(lost)) return;
     for (int64_t tile = block + blocks * (threadIdx.x >> 6); tile < ntiles; tile += blocks * kBlockWaves) {
         for (int64_t row = tile * 16; row < rows && row < tile * 16 + 16; row++) {
             float v = value[row], a = kRoot ? R[row * kE + u] : logit[row];

@@ -901,3 +901,28 @@ def test_leaf_eval_operands_without_split(what):
                 ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)):
         for a, b in zip(got, (priors, value, child_q)):
             assert float((a.double() - b).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("layer", ["fc1", "fc2", "action_fc1"])
+def test_leaf_eval_nan_network(layer):
+    """A NaN weight of the encoder makes every output NaN, one of the action head
+    the priors of every leaf with moves and no value."""
+    import torch
+
+    from hive_neuralnet_amd import hive_gpu
+    from hive_neuralnet_amd.fnn import seeded_large
+    ext = hive_gpu.load_extension()
+    net = seeded_large(8)
+    T = 420
+    st = hive_gpu.random_positions(T, 0, 110, 23)[0]
+    mv, n, feat = ext.generate_legal_moves_and_fnn_features_batch(st, T)
+    plain = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
+    with torch.no_grad():
+        getattr(net, layer).weight[5, 70 if layer == "action_fc1" else 5] = float("nan")
+    priors, value, child_q = ext.fnn_leaf_eval_lists(st, mv, n, feat, T, net)
+    live = torch.arange(256, device="cuda").unsqueeze(0) < n.unsqueeze(1)
+    assert torch.equal(torch.isnan(priors), live)
+    if layer == "action_fc1":
+        assert torch.equal(value, plain[1]) and bool(((child_q - plain[2]).abs() < 1e-5).all())
+    else:
+        assert bool(torch.isnan(value).all()) and torch.equal(torch.isnan(child_q), live)
